@@ -3,7 +3,7 @@
 //
 // Mirrors FW::CudaRaster (src/cudaraster/CudaRaster.cpp): the same state
 // machine, the same validity checks, the same overflow-retry contract
-// (:277-339), per-stage events for getStats (:346-363).  Buffers are plain
+// (:277-339), per-stage times for getStats (:346-363).  Buffers are plain
 // device allocations owned by the context (the reference's lazily migrating
 // FW::Buffer is not needed: inputs are device pointers, surfaces are device
 // buffers).
@@ -243,22 +243,28 @@ Params makeParams(cr_context* ctx, const Geometry& g, int32_t numChunks, const D
   return P;
 }
 
-cr_status launchAll(cr_context* ctx, const Params& P, hipStream_t stream) {
-  CR_HIP(ctx, hipEventRecord(ctx->ev[0], stream));
-  launchReset(P, stream);
+cr_status launchAll(cr_context* ctx, const Params& P, hipStream_t stream, bool reset) {
+  // A captured draw runs when its graph is launched, after whatever other
+  // draws: it clears the block itself and says nothing about its state now.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    cap = hipStreamCaptureStatusNone;
+  }
+  const bool captured = cap != hipStreamCaptureStatusNone;
+  if (reset || captured || !ctx->countersClean || P.prof) launchReset(P, stream);
+  if (!captured && !reset) ctx->countersClean = false;
   launchSetup(P, stream);                       // setup and binning are one kernel
-  CR_HIP(ctx, hipEventRecord(ctx->ev[1], stream));   // (no separate bin stage to bracket)
   launchCoarse(P, stream);
-  CR_HIP(ctx, hipEventRecord(ctx->ev[3], stream));
   launchFine(P, stream);
-  CR_HIP(ctx, hipEventRecord(ctx->ev[4], stream));
   launchFragmentSum(P, stream);
+  launchFinish(P, ctx->hostCountersDev, stream);
   CR_HIP(ctx, hipGetLastError());
-  CR_HIP(ctx, hipMemcpyAsync(ctx->hostCounters, P.counters, sizeof(Counters), hipMemcpyDeviceToHost, stream));
+  if (!captured && !reset) ctx->countersClean = true;
   if (P.prof)
     CR_HIP(ctx, hipMemcpyAsync(ctx->hostProf, P.prof, 2 * kProfCount * sizeof(unsigned long long),
                                hipMemcpyDeviceToHost, stream));
-  ctx->evRecorded = true;
+  ctx->drawn = true;
   ctx->lastProfiled = P.prof != nullptr;
   return CR_OK;
 }
@@ -317,7 +323,7 @@ cr_status drawImpl(cr_context* ctx, hipStream_t stream, bool sync) {
     st = ensureBuffers(ctx, g, numChunks);
     if (st != CR_OK) return st;
     Params P = makeParams(ctx, g, numChunks, contextBuffers(ctx));
-    st = launchAll(ctx, P, stream);
+    st = launchAll(ctx, P, stream, false);
     if (st != CR_OK) return st;
     if (!sync) {
       // Waiting on this event (not on the stream) lets cr_draw_check return
@@ -363,7 +369,10 @@ cr_status cr_context_create(cr_context** out) {
   if (e == hipSuccess) e = hipHostMalloc((void**)&ctx->hostCounters, sizeof(Counters), hipHostMallocDefault);
   if (e == hipSuccess)
     e = hipHostMalloc((void**)&ctx->hostProf, 2 * kProfCount * sizeof(unsigned long long), hipHostMallocDefault);
-  for (int i = 0; i < 5 && e == hipSuccess; i++) e = hipEventCreate(&ctx->ev[i]);
+  if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&ctx->hostCountersDev, ctx->hostCounters, 0);
+  int khz = 0;
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device);
+  if (khz > 0) ctx->clockSeconds = 1e-3 / khz;
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->evPending, hipEventDisableTiming);
   if (e != hipSuccess) {
     cr_context_destroy(ctx);
@@ -386,8 +395,6 @@ cr_status cr_context_destroy(cr_context* ctx) {
     b->release();
   if (ctx->hostCounters) (void)hipHostFree(ctx->hostCounters);
   if (ctx->hostProf) (void)hipHostFree(ctx->hostProf);
-  for (int i = 0; i < 5; i++)
-    if (ctx->ev[i]) (void)hipEventDestroy(ctx->ev[i]);
   if (ctx->evPending) (void)hipEventDestroy(ctx->evPending);
   delete ctx;
   return CR_OK;
@@ -603,19 +610,19 @@ cr_status cr_reserve(cr_context* ctx, int64_t maxSubtris, int64_t maxBin, int64_
 cr_status cr_get_stats(cr_context* ctx, cr_stats* out) {
   if (!ctx || !out) return fail(ctx, CR_ERR_INVALID, "cr_get_stats: NULL argument");
   memset(out, 0, sizeof(*out));
-  if (!ctx->evRecorded) return CR_OK;
-  CR_HIP(ctx, hipEventSynchronize(ctx->ev[4]));
-  // Binning runs inside the setup kernel: its time is part of setup_time and
-  // bin_time is 0 (an extra event pair between the two would cost the GPU
-  // a few microseconds per draw).
-  float setupMs = 0.0f, coarseMs = 0.0f, fineMs = 0.0f;
-  CR_HIP(ctx, hipEventElapsedTime(&setupMs, ctx->ev[0], ctx->ev[1]));
-  CR_HIP(ctx, hipEventElapsedTime(&coarseMs, ctx->ev[1], ctx->ev[3]));
-  CR_HIP(ctx, hipEventElapsedTime(&fineMs, ctx->ev[3], ctx->ev[4]));
-  out->setup_time = setupMs * 1e-3f;
+  if (!ctx->drawn) return CR_OK;
+  if (ctx->pending) CR_HIP(ctx, hipEventSynchronize(ctx->evPending));
+  // Each stage lasts until the next one starts.  Binning runs inside the
+  // setup kernel: its time is part of setup_time and bin_time is 0.  (A draw
+  // without triangles has no setup stage and no setup stamp.)
+  const uint64_t* s = ctx->hostCounters->stamp;
+  auto seconds = [&](uint64_t from, uint64_t to) {
+    return from != 0 && to > from ? (float)((double)(to - from) * ctx->clockSeconds) : 0.0f;
+  };
+  out->setup_time = seconds(s[kStampSetup], s[kStampCoarse]);
   out->bin_time = 0.0f;
-  out->coarse_time = coarseMs * 1e-3f;
-  out->fine_time = fineMs * 1e-3f;
+  out->coarse_time = seconds(s[kStampCoarse], s[kStampFine]);
+  out->fine_time = seconds(s[kStampFine], s[kStampEnd]);
   return CR_OK;
 }
 

@@ -69,7 +69,9 @@ struct cr_batch {
   std::vector<ViewState> views;
   DevBuf triSubtris, triHeader, triData, subtriTri, chunkBase, binCnt, binOff, binList;
   DevBuf tileStart, tileCount, tileList, tileSegNext, counters, saved;
-  Counters* hostCounters = nullptr;   // pinned, one block per view
+  Counters* hostCounters = nullptr;   // pinned, one block per view, written by the draws' finish kernels
+  Counters* hostCountersDev = nullptr;   // their device address
+  bool countersClean = false;         // every view's last draw was queued whole: it leaves its counters cleared
   Tables groups[kMaxGroups];          // views split into cost-balanced groups, one launch chain each
   int numGroups = 1;
   Tables subset;                      // views re-drawn after an overflow
@@ -83,7 +85,6 @@ struct cr_batch {
   hipStream_t capStream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
   float lastMs = 0.0f, tunedMs = 0.0f;
   int64_t retries = 0;
   size_t reserved = 0;
@@ -125,7 +126,9 @@ cr_status layout(cr_batch* b) {
   CR_HIP(ctx, b->tileCount.ensure(nTile * 4));
   CR_HIP(ctx, b->tileList.ensure(nTileList * 4));
   CR_HIP(ctx, b->tileSegNext.ensure(std::max<size_t>(nTileList >> kTileSegLog2, 1) * 8));
+  const void* before = b->counters.ptr;
   CR_HIP(ctx, b->counters.ensure(b->views.size() * sizeof(Counters)));
+  if (b->counters.ptr != before) b->countersClean = false;
   b->reserved = b->triSubtris.bytes + b->triHeader.bytes + b->triData.bytes + b->subtriTri.bytes +
                 b->chunkBase.bytes + b->binCnt.bytes + b->binOff.bytes + b->binList.bytes + b->tileStart.bytes +
                 b->tileCount.bytes + b->tileList.bytes + b->tileSegNext.bytes + b->counters.bytes;
@@ -300,12 +303,12 @@ cr_status buildAll(cr_batch* b) {
 cr_status launchTables(cr_batch* b, const Tables& T, hipStream_t stream) {
   const Params* pv = T.params.as<Params>();
   const int32_t* s = T.starts.as<int32_t>();
-  launchResetBatch(pv, T.n, stream);
   launchSetupBatch(pv, s + T.setup.ofs, s + T.setup.orderOfs, T.setup.n, T.setup.blocks, stream);
   launchCoarseBatch(b->coarseThreads, pv, s + T.coarse.ofs, s + T.coarse.orderOfs, T.coarse.n, T.coarse.blocks,
                     stream);
   for (const Tables::Stage& f : T.fine)
     launchFineBatch(f.variant, b->tilesPerGroup, b->banded, pv, s + f.ofs, s + f.orderOfs, f.n, f.blocks, stream);
+  launchFinishBatch(pv, T.n, b->counters.as<Counters>(), b->hostCountersDev, stream);
   CR_HIP(b->ctx, hipGetLastError());
   return CR_OK;
 }
@@ -341,18 +344,20 @@ cr_status capture(cr_batch* b) {
   return CR_OK;
 }
 
-cr_status readCounters(cr_batch* b, hipStream_t stream) {
-  CR_HIP(b->ctx, hipMemcpyAsync(b->hostCounters, b->counters.ptr, b->views.size() * sizeof(Counters),
-                                hipMemcpyDeviceToHost, stream));
-  CR_HIP(b->ctx, hipStreamSynchronize(stream));
-  return CR_OK;
-}
-
 cr_status prepare(cr_batch* b) {
   if (b->laidOut) return CR_OK;
   cr_status st = layout(b);
   if (st != CR_OK) return st;
   return buildAll(b);
+}
+
+// Clears the counters of every view unless the draw before left them so.
+cr_status clearCounters(cr_batch* b, hipStream_t stream) {
+  if (b->countersClean) return CR_OK;
+  for (int g = 0; g < b->numGroups; g++)
+    launchResetBatch(b->groups[g].params.as<Params>(), b->groups[g].n, stream);
+  CR_HIP(b->ctx, hipGetLastError());
+  return CR_OK;
 }
 
 // Grows the capacities of every view whose counters overflowed and re-draws
@@ -381,9 +386,13 @@ cr_status settleOverflow(cr_batch* b, hipStream_t stream) {
     cr_status st = layout(b);
     if (st == CR_OK) st = buildAll(b);
     if (st == CR_OK) st = buildTables(b, b->subset, over);
-    if (st == CR_OK) st = launchTables(b, b->subset, stream);
-    if (st == CR_OK) st = readCounters(b, stream);
+    if (st == CR_OK) st = clearCounters(b, stream);
     if (st != CR_OK) return st;
+    b->countersClean = false;
+    st = launchTables(b, b->subset, stream);
+    if (st != CR_OK) return st;
+    b->countersClean = true;
+    CR_HIP(b->ctx, hipStreamSynchronize(stream));
   }
 }
 
@@ -397,17 +406,26 @@ cr_status drawBatch(cr_batch* b, hipStream_t stream, bool graph) {
     st = capture(b);
     if (st != CR_OK) return st;
   }
-  CR_HIP(ctx, hipEventRecord(b->ev0, stream));
+  st = clearCounters(b, stream);
+  if (st != CR_OK) return st;
+  b->countersClean = false;
   if (graph) {
     CR_HIP(ctx, hipGraphLaunch(b->exec, stream));
   } else {
     st = launchAllGroups(b, stream);
     if (st != CR_OK) return st;
   }
-  CR_HIP(ctx, hipEventRecord(b->ev1, stream));
-  st = readCounters(b, stream);
-  if (st != CR_OK) return st;
-  CR_HIP(ctx, hipEventElapsedTime(&b->lastMs, b->ev0, b->ev1));
+  b->countersClean = true;
+  CR_HIP(ctx, hipStreamSynchronize(stream));
+  // GPU time: the first stage's start to the last view's end.
+  uint64_t first = UINT64_MAX, last = 0;
+  for (size_t i = 0; i < b->views.size(); i++) {
+    const uint64_t* s = b->hostCounters[i].stamp;
+    for (int k = 0; k < kStampCount; k++)
+      if (s[k] != 0) first = std::min(first, s[k]);
+    last = std::max(last, s[kStampEnd]);
+  }
+  b->lastMs = last > first ? (float)((double)(last - first) * ctx->clockSeconds * 1e3) : 0.0f;
   return settleOverflow(b, stream);
 }
 
@@ -492,8 +510,7 @@ cr_status cr_batch_create(cr_context* ctx, const cr_view* views, int32_t numView
   if (e == hipSuccess) e = hipHostMalloc((void**)&b->hostCounters, std::max<size_t>(numViews, 1) * sizeof(Counters),
                                          hipHostMallocDefault);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->capStream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipEventCreate(&b->ev0);
-  if (e == hipSuccess) e = hipEventCreate(&b->ev1);
+  if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&b->hostCountersDev, b->hostCounters, 0);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->evFork, hipEventDisableTiming);
   for (int g = 1; g < kMaxGroups && e == hipSuccess; g++) {
     e = hipStreamCreateWithFlags(&b->side[g], hipStreamNonBlocking);
@@ -530,8 +547,6 @@ cr_status cr_batch_destroy(cr_batch* b) {
     if (b->evJoin[g]) (void)hipEventDestroy(b->evJoin[g]);
   }
   if (b->evFork) (void)hipEventDestroy(b->evFork);
-  if (b->ev0) (void)hipEventDestroy(b->ev0);
-  if (b->ev1) (void)hipEventDestroy(b->ev1);
   delete b;
   return CR_OK;
 }

@@ -25,6 +25,8 @@
 // the segment starts, one round ahead.  Large boxes are shared out over the
 // workgroup's waves through an LDS queue.  Binning never changes the image;
 // the fine stage is exact.
+#include <cstddef>
+
 #include "cr_device.h"
 
 namespace crhip {
@@ -70,14 +72,42 @@ __device__ __forceinline__ uint32_t blockScanC(uint32_t v, uint32_t* sums, uint3
 }
 
 // Clears the counter block (and a profiling draw's profile counters) with
-// plain stores: graph-safe, no memset node.
-__global__ void __launch_bounds__(64) resetCountersKernel(Counters* c, uint32_t numTris, unsigned long long* prof) {
+// plain stores: graph-safe, no memset node.  Only for draws that cannot rely
+// on the draw before them having left the block cleared.
+__global__ void __launch_bounds__(64) resetCountersKernel(Counters* c, unsigned long long* prof) {
   uint32_t* w = reinterpret_cast<uint32_t*>(c);
   for (int i = threadIdx.x; i < (int)(sizeof(Counters) / 4); i += 64) w[i] = 0;
   if (prof != nullptr)
     for (int i = threadIdx.x; i < 2 * kProfCount; i += 64) prof[i] = 0;
-  __syncthreads();
-  if (threadIdx.x == 0) c->numSubtris = numTris;
+}
+
+// End of a draw: the counter block into its host copy (pinned memory,
+// written by the kernel), the end stamp, and the block cleared for the next
+// draw.  One small kernel in the place of a reset kernel before the draw and
+// a copy after it; one wave, a word per lane.
+__device__ __forceinline__ void finishBody(Counters* dev, Counters* host, uint32_t numTris) {
+  static_assert(sizeof(Counters) == 64 * 4, "one word per lane");
+  const uint64_t now = wall_clock64();
+  const int i = (int)threadIdx.x;
+  uint32_t* d = reinterpret_cast<uint32_t*>(dev);
+  uint32_t v = d[i];
+  d[i] = 0;
+  constexpr int kEndWord = (int)(offsetof(Counters, stamp) / 4) + 2 * kStampEnd;
+  if (i == (int)(offsetof(Counters, numSubtris) / 4)) v += numTris;
+  if (i == kEndWord) v = (uint32_t)now;
+  if (i == kEndWord + 1) v = (uint32_t)(now >> 32);
+  reinterpret_cast<uint32_t*>(host)[i] = v;
+}
+
+__global__ void __launch_bounds__(64) finishKernel(Counters* dev, Counters* host, uint32_t numTris) {
+  finishBody(dev, host, numTris);
+}
+
+// One workgroup per view of a batch.
+__global__ void __launch_bounds__(64) finishBatchKernel(const Params* __restrict__ views,
+                                                        const Counters* devBase, Counters* hostBase) {
+  const Params& P = views[blockIdx.x];
+  finishBody(P.counters, hostBase + (P.counters - devBase), (uint32_t)P.numTris);
 }
 
 // Per-lane tile test data of one triangle inside bin (bx, by).
@@ -338,6 +368,7 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
   // Profiling draws: entries, rounds, emits, tiles with emits, entries per case.
   __shared__ uint32_t sProf[8];
 
+  if (bin == 0) stampStage(P, kStampCoarse);
   if (P.counters->overflow & 3u) return;
   const bool prof = P.prof != nullptr;
   if (prof && threadIdx.x < 8) sProf[threadIdx.x] = 0;
@@ -669,12 +700,20 @@ __global__ void __launch_bounds__(64) resetBatchKernel(const Params* __restrict_
   const Params& P = views[blockIdx.x];
   uint32_t* w = reinterpret_cast<uint32_t*>(P.counters);
   for (int i = threadIdx.x; i < (int)(sizeof(Counters) / 4); i += 64) w[i] = 0;
-  __syncthreads();
-  if (threadIdx.x == 0) P.counters->numSubtris = (uint32_t)P.numTris;
 }
 
 void launchReset(const Params& P, hipStream_t stream) {
-  hipLaunchKernelGGL(resetCountersKernel, dim3(1), dim3(64), 0, stream, P.counters, (uint32_t)P.numTris, P.prof);
+  hipLaunchKernelGGL(resetCountersKernel, dim3(1), dim3(64), 0, stream, P.counters, P.prof);
+}
+
+void launchFinish(const Params& P, Counters* host, hipStream_t stream) {
+  hipLaunchKernelGGL(finishKernel, dim3(1), dim3(64), 0, stream, P.counters, host, (uint32_t)P.numTris);
+}
+
+void launchFinishBatch(const Params* views, int numViews, const Counters* devBase, Counters* hostBase,
+                       hipStream_t stream) {
+  if (numViews <= 0) return;
+  hipLaunchKernelGGL(finishBatchKernel, dim3(numViews), dim3(64), 0, stream, views, devBase, hostBase);
 }
 
 int coarseShapeFor(const Params& P) {

@@ -68,9 +68,17 @@ struct TriData {         // CRTriangleData
 static_assert(sizeof(Header) == 16, "header layout");
 static_assert(sizeof(TriData) == 64, "data layout");
 
-// Device counters; one 256-byte block per context.
+// Stage times: the first workgroup of a stage (and the finish kernel) notes
+// the device's wall clock in the counter block.  Timed events around the stages
+// put four more packets into the stream, each waiting for the kernel before
+// it: 17 us of the 75 us that a draw of 12 triangles took with them, a reset
+// kernel and a counter copy, 55 us without (1M triangles: 324 -> 307 us).
+enum Stamp : int { kStampSetup = 0, kStampCoarse, kStampFine, kStampEnd, kStampCount };
+
+// Device counters; one 256-byte block per context.  All zero between draws:
+// the finish kernel hands them to the host and clears them.
 struct Counters {
-  uint32_t numSubtris;     // slot allocator for clipped subtriangles (starts at numTris)
+  uint32_t numSubtris;     // clipped subtriangles' slots in use past numTris (host copy: plus numTris)
   uint32_t tileEntries;    // tile-list allocator: entries reserved, in whole 32-entry segments
   uint32_t overflow;       // bit 0 subtris, bit 1 bin entries, bit 2 tile entries
   uint32_t binEntries;     // bin-queue entry allocator
@@ -78,7 +86,8 @@ struct Counters {
   uint32_t pad0[3];
   uint64_t fragments;      // (subtriangle, pixel) pairs with >= 1 covered sample
   uint64_t visibleSubtris; // subtriangles that survive setup (counting draws only)
-  uint64_t pad[26];
+  uint64_t stamp[kStampCount];   // wall clock at the stages' starts and the draw's end (0: stage not run)
+  uint64_t pad[26 - kStampCount];
 };
 static_assert(sizeof(Counters) == 256, "counter block");
 
@@ -306,8 +315,14 @@ __host__ __device__ inline int selectCentroid(int s, uint32_t mask) {
   return best;
 }
 
+// Called by every thread of a stage's workgroup 0.
+__device__ __forceinline__ void stampStage(const Params& P, Stamp s) {
+  if (threadIdx.x == 0) P.counters->stamp[s] = wall_clock64();
+}
+
 // Host-side launchers, one per stage file.
 void launchReset(const Params& P, hipStream_t stream);
+void launchFinish(const Params& P, Counters* host, hipStream_t stream);
 void launchSetup(const Params& P, hipStream_t stream);     // setup + bin
 void launchCoarse(const Params& P, hipStream_t stream);
 void launchFine(const Params& P, hipStream_t stream);
@@ -319,6 +334,9 @@ constexpr int kSetupChunkTris = 1024;
 // its own order: the k-th listed view is views[order[k]] and owns the
 // workgroups [blockStart[k], blockStart[k+1]).
 void launchResetBatch(const Params* views, int numViews, hipStream_t stream);
+// devBase, hostBase: the batch's counter blocks and their host copies.
+void launchFinishBatch(const Params* views, int numViews, const Counters* devBase, Counters* hostBase,
+                       hipStream_t stream);
 void launchSetupBatch(const Params* views, const int32_t* blockStart, const int32_t* order, int numViews,
                       int totalBlocks, hipStream_t stream);
 void launchCoarseBatch(int threads, const Params* views, const int32_t* blockStart, const int32_t* order,

@@ -207,6 +207,7 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
   uint32_t* __restrict__ triid = P.triid;
   const int32_t blend = BL >= 0 ? BL : P.blend;
 
+  if (group == 0) stampStage(P, kStampFine);
   const int lane = threadIdx.x & 63;
   // Wave-uniform, so the tile's coordinates and addresses are scalars.
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));

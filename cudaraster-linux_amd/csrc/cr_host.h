@@ -134,9 +134,10 @@ cr_status validateDraw(cr_context* ctx);
 DrawBuffers contextBuffers(cr_context* ctx);
 // Kernel parameters of the context's current state over buffers B.
 crhip::Params makeParams(cr_context* ctx, const Geometry& g, int32_t numChunks, const DrawBuffers& B);
-// Reset, setup+bin, coarse and fine launches with the stage events, then the
-// counter block's copy into ctx->hostCounters, all on `stream`.
-cr_status launchAll(cr_context* ctx, const crhip::Params& P, hipStream_t stream);
+// Setup+bin, coarse, fine and finish launches on `stream`; the last one puts
+// the counters into ctx->hostCounters and clears the block.  reset: clear the
+// block before the draw too (a block that other draws may have left in use).
+cr_status launchAll(cr_context* ctx, const crhip::Params& P, hipStream_t stream, bool reset);
 // Copies the read-back counters into ctx->last; returns their overflow bits.
 uint32_t recordCounters(cr_context* ctx);
 // Looks up this device's copy of the no-allocation draw's fixed scratch
@@ -177,12 +178,14 @@ struct cr_context {
   crhost::DevBuf tileStart, tileCount, tileList, tileSegNext, tileFrags, chunkSubtris;
   crhost::DevBuf counters, profBuf;
   crhost::DevBuf interpAcc;                  // fixed-point gradient accumulators (deterministic backward)
-  crhip::Counters* hostCounters = nullptr;   // pinned
+  crhip::Counters* hostCounters = nullptr;   // pinned, written by the draw's finish kernel
+  crhip::Counters* hostCountersDev = nullptr;   // its device address
+  bool countersClean = false;                // the last draw of `counters` was queued whole: it leaves them cleared
   unsigned long long* hostProf = nullptr;    // pinned, 2 * kProfCount
   cr_profile_counters lastProf{};
   bool lastProfiled = false;                 // the last launch recorded profile counters
-  hipEvent_t ev[5] = {};
-  bool evRecorded = false;
+  bool drawn = false;                 // hostCounters hold (or will hold) a draw's stamps
+  double clockSeconds = 1e-8;         // one tick of the device's wall clock
   hipStream_t pendingStream = nullptr;
   hipEvent_t evPending = nullptr;     // after an asynchronous draw's counter readback
   bool pending = false;

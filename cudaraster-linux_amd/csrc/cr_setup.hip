@@ -273,7 +273,7 @@ __device__ __noinline__ int setupClipped(const ClipCtx P, int t, int3 vidx, floa
 
   int base = t;
   if (numSub > 1) {
-    base = (int)atomicAdd(&P.counters->numSubtris, (uint32_t)numSub);
+    base = P.numTris + (int)atomicAdd(&P.counters->numSubtris, (uint32_t)numSub);
     P.triHeader[t].misc = (uint32_t)base;
     if (base + numSub > P.maxSubtris) {
       atomicOr(&P.counters->overflow, 1u);
@@ -457,6 +457,7 @@ __device__ __forceinline__ void setupBinBody(const Params& P, const int chunk) {
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t = chunk * kSetupChunk + threadIdx.x;
+  if (chunk == 0) stampStage(P, kStampSetup);
 
   // ---- setup ---------------------------------------------------------------
   int base = t, k = 0, why = kSetupDropped;
