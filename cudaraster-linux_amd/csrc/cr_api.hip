@@ -15,6 +15,7 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <vector>
 
 #include "cr/cr.h"
 #include "cr_device.h"
@@ -349,7 +350,7 @@ cr_status drawImpl(cr_context* ctx, hipStream_t stream, bool sync) {
 
 extern "C" {
 
-int32_t cr_abi_version(void) { return (1 << 16) | 6; }
+int32_t cr_abi_version(void) { return (1 << 16) | 7; }
 
 const char* cr_last_error(const cr_context* ctx) { return ctx ? ctx->err.c_str() : g_lastError.c_str(); }
 
@@ -725,68 +726,171 @@ cr_status cr_get_profile_counters(cr_context* ctx, cr_profile_counters* out) {
   return CR_OK;
 }
 
+namespace {
+
+// What the forward calls ask of a view's buffers.  (Without vertices the
+// kernels read no position or attribute: an empty view may pass NULL for
+// them.)
+bool forwardBuffersOk(const cr_interp_view& v, int32_t numChannels) {
+  return numChannels >= 0 && v.num_vertices >= 0 && v.num_tris >= 0 && v.num_tris <= INT32_MAX &&
+         !(numChannels > 0 && v.num_vertices > 0 && !v.attr) && !(v.num_tris > 0 && (!v.pos || !v.tris)) &&
+         !((uintptr_t)v.pos & 15) && !((uintptr_t)v.tris & 3);
+}
+
+InterpView interpView(const cr_interp_view& v, const uint32_t* ids) {
+  InterpView V{};
+  V.ids = ids;
+  V.pos = v.pos;
+  V.attr = v.attr;
+  V.tris = v.tris;
+  V.out = v.out;
+  V.triImage = v.tri_image;
+  V.gradOut = v.grad_out;
+  V.gradPos = v.grad_pos;
+  V.gradAttr = v.grad_attr;
+  V.numVertices = v.num_vertices;
+  V.numTris = (int32_t)v.num_tris;
+  return V;
+}
+
+cr_status interpolateViews(cr_context* ctx, const char* name, const cr_interp_view* views, int32_t numViews,
+                           int32_t numChannels, void* stream) {
+  std::vector<InterpView> table;
+  try {
+    table.reserve((size_t)numViews);
+  } catch (const std::bad_alloc&) {
+    return fail(ctx, CR_ERR_NOMEM, "out of host memory");
+  }
+  for (int32_t k = 0; k < numViews; k++) {
+    const cr_interp_view& v = views[k];
+    if (!v.tri_id || !v.out) return fail(ctx, CR_ERR_INVALID, "%s: NULL argument", name);
+    if (v.tri_id->format != CR_FORMAT_TRIANGLE_ID || v.tri_id->samples != 1)
+      return fail(ctx, CR_ERR_INVALID, "%s: needs a single-sample CR_FORMAT_TRIANGLE_ID surface", name);
+    if (!forwardBuffersOk(v, numChannels)) return fail(ctx, CR_ERR_INVALID, "%s: bad buffers or counts", name);
+    if (v.tri_id->width != views[0].tri_id->width || v.tri_id->height != views[0].tri_id->height)
+      return fail(ctx, CR_ERR_INVALID, "%s: the views differ in resolution", name);
+    table.push_back(interpView(v, v.tri_id->dev));
+  }
+  if (numViews == 0) return CR_OK;
+  const cr_surface* s = views[0].tri_id;
+  InterpGeom G{s->width, s->height, s->textureW, numChannels};
+  CR_HIP(ctx, hipSetDevice(ctx->device));
+  launchInterpForward(G, table.data(), numViews, static_cast<hipStream_t>(stream));
+  CR_HIP(ctx, hipGetLastError());
+  return CR_OK;
+}
+
+// Fixed-point accumulators of the views that share a launch are at most this
+// large (a single view may need more).
+constexpr size_t kInterpAccBytes = (size_t)1 << 29;
+
+cr_status interpolateBackward(cr_context* ctx, const char* name, bool deterministic, const cr_interp_view* views,
+                              int32_t numViews, int32_t width, int32_t height, int32_t numChannels, void* stream) {
+  std::vector<InterpView> table;
+  try {
+    table.reserve((size_t)numViews);
+  } catch (const std::bad_alloc&) {
+    return fail(ctx, CR_ERR_NOMEM, "out of host memory");
+  }
+  for (int32_t k = 0; k < numViews; k++) {
+    const cr_interp_view& v = views[k];
+    // (Without vertices there is no gradient to write and no attribute to read.)
+    if (!v.tri_image || !v.grad_out ||
+        (v.num_vertices > 0 && (!v.grad_pos || (numChannels > 0 && (!v.attr || !v.grad_attr)))))
+      return fail(ctx, CR_ERR_INVALID, "%s: NULL argument", name);
+    if (width <= 0 || height <= 0 || width > kMaxViewport || height > kMaxViewport || numChannels < 0 ||
+        v.num_vertices < 0 || v.num_tris < 0 || v.num_tris > INT32_MAX || (v.num_tris > 0 && (!v.pos || !v.tris)) ||
+        ((uintptr_t)v.pos & 15) || ((uintptr_t)v.tris & 3))
+      return fail(ctx, CR_ERR_INVALID, "%s: bad sizes or buffers", name);
+    table.push_back(interpView(v, nullptr));
+  }
+  CR_HIP(ctx, hipSetDevice(ctx->device));
+  InterpGeom G{width, height, width, numChannels};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (!deterministic) {
+    launchInterpBackward(G, table.data(), numViews, s);
+  } else {
+    for (int32_t k0 = 0, k1; k0 < numViews; k0 = k1) {
+      // As many views as the accumulators' bound admits, at least one.
+      size_t bytes = 0;
+      for (k1 = k0; k1 < numViews && k1 - k0 < kInterpViews; k1++) {
+        const size_t b = (size_t)std::max<int64_t>(table[k1].numVertices * (4 + (int64_t)numChannels), 1) * 16;
+        if (k1 > k0 && bytes + b > kInterpAccBytes) break;
+        bytes += b;
+      }
+      CR_HIP(ctx, ctx->interpAcc.ensure(bytes));
+      unsigned long long* acc = ctx->interpAcc.as<unsigned long long>();
+      for (int32_t k = k0; k < k1; k++) {
+        table[k].acc = acc;
+        acc += 2 * std::max<int64_t>(table[k].numVertices * (4 + (int64_t)numChannels), 1);
+      }
+      launchInterpBackward(G, table.data() + k0, k1 - k0, s);
+    }
+  }
+  CR_HIP(ctx, hipGetLastError());
+  return CR_OK;
+}
+
+}  // namespace
+
 cr_status cr_interpolate(cr_context* ctx, const cr_surface* triId, const float* pos, int64_t numVertices,
                          const float* attr, int32_t numChannels, const int32_t* tris, int32_t numTris, float* out,
                          int32_t* triImage, void* stream) {
-  if (!ctx || !triId || !out) return fail(ctx, CR_ERR_INVALID, "cr_interpolate: NULL argument");
-  if (triId->format != CR_FORMAT_TRIANGLE_ID || triId->samples != 1)
-    return fail(ctx, CR_ERR_INVALID, "cr_interpolate: needs a single-sample CR_FORMAT_TRIANGLE_ID surface");
-  // (Without vertices the kernels read no position or attribute: an empty
-  // view may pass NULL for them.)
-  if (numChannels < 0 || numVertices < 0 || numTris < 0 || (numChannels > 0 && numVertices > 0 && !attr) ||
-      (numTris > 0 && (!pos || !tris)) || ((uintptr_t)pos & 15) || ((uintptr_t)tris & 3))
-    return fail(ctx, CR_ERR_INVALID, "cr_interpolate: bad buffers or counts");
-  InterpGeom G{triId->width, triId->height, triId->textureW, numChannels, numTris, numVertices};
-  CR_HIP(ctx, hipSetDevice(ctx->device));
-  launchInterpForward(G, triId->dev, pos, attr, tris, out, triImage, static_cast<hipStream_t>(stream));
-  CR_HIP(ctx, hipGetLastError());
-  return CR_OK;
+  if (!ctx) return fail(ctx, CR_ERR_INVALID, "cr_interpolate: NULL argument");
+  cr_interp_view v{};
+  v.tri_id = triId;
+  v.pos = pos;
+  v.num_vertices = numVertices;
+  v.attr = attr;
+  v.tris = tris;
+  v.num_tris = numTris;
+  v.out = out;
+  v.tri_image = triImage;
+  return interpolateViews(ctx, "cr_interpolate", &v, 1, numChannels, stream);
 }
 
 cr_status cr_interpolate_ids(cr_context* ctx, const int32_t* triImage, int32_t width, int32_t height,
                              const float* pos, int64_t numVertices, const float* attr, int32_t numChannels,
                              const int32_t* tris, int32_t numTris, float* out, void* stream) {
   if (!ctx || !triImage || !out) return fail(ctx, CR_ERR_INVALID, "cr_interpolate_ids: NULL argument");
-  if (width <= 0 || height <= 0 || width > kMaxViewport || height > kMaxViewport || numChannels < 0 ||
-      numVertices < 0 || numTris < 0 || (numChannels > 0 && numVertices > 0 && !attr) ||
-      (numTris > 0 && (!pos || !tris)) || ((uintptr_t)pos & 15) || ((uintptr_t)tris & 3) ||
-      ((uintptr_t)triImage & 3))
+  cr_interp_view v{};
+  v.pos = pos;
+  v.num_vertices = numVertices;
+  v.attr = attr;
+  v.tris = tris;
+  v.num_tris = numTris;
+  v.out = out;
+  if (width <= 0 || height <= 0 || width > kMaxViewport || height > kMaxViewport ||
+      !forwardBuffersOk(v, numChannels) || ((uintptr_t)triImage & 3))
     return fail(ctx, CR_ERR_INVALID, "cr_interpolate_ids: bad sizes or buffers");
   // An int32 id image is a single-sample id surface with a pitch of `width`
   // texels (-1 reads as 0xFFFFFFFF: no triangle).
-  InterpGeom G{width, height, width, numChannels, numTris, numVertices};
+  InterpGeom G{width, height, width, numChannels};
+  const InterpView V = interpView(v, reinterpret_cast<const uint32_t*>(triImage));
   CR_HIP(ctx, hipSetDevice(ctx->device));
-  launchInterpForward(G, reinterpret_cast<const uint32_t*>(triImage), pos, attr, tris, out, nullptr,
-                      static_cast<hipStream_t>(stream));
+  launchInterpForward(G, &V, 1, static_cast<hipStream_t>(stream));
   CR_HIP(ctx, hipGetLastError());
   return CR_OK;
 }
 
 namespace {
 
-cr_status interpolateBackward(cr_context* ctx, const char* name, bool deterministic, const int32_t* triImage,
-                              int32_t width, int32_t height, const float* pos, int64_t numVertices,
-                              const float* attr, int32_t numChannels, const int32_t* tris, int32_t numTris,
-                              const float* gradOut, float* gradPos, float* gradAttr, void* stream) {
-  // (Without vertices there is no gradient to write and no attribute to read.)
-  if (!ctx || !triImage || !gradOut || (numVertices > 0 && (!gradPos || (numChannels > 0 && (!attr || !gradAttr)))))
-    return fail(ctx, CR_ERR_INVALID, "%s: NULL argument", name);
-  if (width <= 0 || height <= 0 || width > kMaxViewport || height > kMaxViewport || numChannels < 0 ||
-      numVertices < 0 || numTris < 0 || (numTris > 0 && (!pos || !tris)) || ((uintptr_t)pos & 15) ||
-      ((uintptr_t)tris & 3))
-    return fail(ctx, CR_ERR_INVALID, "%s: bad sizes or buffers", name);
-  CR_HIP(ctx, hipSetDevice(ctx->device));
-  InterpGeom G{width, height, width, numChannels, numTris, numVertices};
-  unsigned long long* acc = nullptr;
-  if (deterministic) {
-    const int64_t words = 2 * numVertices * (4 + (int64_t)numChannels);
-    CR_HIP(ctx, ctx->interpAcc.ensure((size_t)std::max<int64_t>(words, 1) * 8));
-    acc = ctx->interpAcc.as<unsigned long long>();
-  }
-  launchInterpBackward(G, triImage, pos, attr, tris, gradOut, gradPos, gradAttr, acc,
-                       static_cast<hipStream_t>(stream));
-  CR_HIP(ctx, hipGetLastError());
-  return CR_OK;
+cr_status interpolateBackwardOne(cr_context* ctx, const char* name, bool deterministic, const int32_t* triImage,
+                                 int32_t width, int32_t height, const float* pos, int64_t numVertices,
+                                 const float* attr, int32_t numChannels, const int32_t* tris, int32_t numTris,
+                                 const float* gradOut, float* gradPos, float* gradAttr, void* stream) {
+  if (!ctx) return fail(ctx, CR_ERR_INVALID, "%s: NULL argument", name);
+  cr_interp_view v{};
+  v.pos = pos;
+  v.num_vertices = numVertices;
+  v.attr = attr;
+  v.tris = tris;
+  v.num_tris = numTris;
+  v.tri_image = const_cast<int32_t*>(triImage);
+  v.grad_out = gradOut;
+  v.grad_pos = gradPos;
+  v.grad_attr = gradAttr;
+  return interpolateBackward(ctx, name, deterministic, &v, 1, width, height, numChannels, stream);
 }
 
 }  // namespace
@@ -795,8 +899,8 @@ cr_status cr_interpolate_backward(cr_context* ctx, const int32_t* triImage, int3
                                   const float* pos, int64_t numVertices, const float* attr, int32_t numChannels,
                                   const int32_t* tris, int32_t numTris, const float* gradOut, float* gradPos,
                                   float* gradAttr, void* stream) {
-  return interpolateBackward(ctx, "cr_interpolate_backward", false, triImage, width, height, pos, numVertices,
-                             attr, numChannels, tris, numTris, gradOut, gradPos, gradAttr, stream);
+  return interpolateBackwardOne(ctx, "cr_interpolate_backward", false, triImage, width, height, pos, numVertices,
+                                attr, numChannels, tris, numTris, gradOut, gradPos, gradAttr, stream);
 }
 
 cr_status cr_interpolate_backward_deterministic(cr_context* ctx, const int32_t* triImage, int32_t width,
@@ -804,8 +908,23 @@ cr_status cr_interpolate_backward_deterministic(cr_context* ctx, const int32_t* 
                                                 const float* attr, int32_t numChannels, const int32_t* tris,
                                                 int32_t numTris, const float* gradOut, float* gradPos,
                                                 float* gradAttr, void* stream) {
-  return interpolateBackward(ctx, "cr_interpolate_backward_deterministic", true, triImage, width, height, pos,
-                             numVertices, attr, numChannels, tris, numTris, gradOut, gradPos, gradAttr, stream);
+  return interpolateBackwardOne(ctx, "cr_interpolate_backward_deterministic", true, triImage, width, height, pos,
+                                numVertices, attr, numChannels, tris, numTris, gradOut, gradPos, gradAttr, stream);
+}
+
+cr_status cr_interpolate_views(cr_context* ctx, const cr_interp_view* views, int32_t numViews, int32_t numChannels,
+                               void* stream) {
+  if (!ctx || numViews < 0 || (numViews > 0 && !views))
+    return fail(ctx, CR_ERR_INVALID, "cr_interpolate_views: NULL argument");
+  return interpolateViews(ctx, "cr_interpolate_views", views, numViews, numChannels, stream);
+}
+
+cr_status cr_interpolate_views_backward(cr_context* ctx, const cr_interp_view* views, int32_t numViews, int32_t width,
+                                        int32_t height, int32_t numChannels, int32_t deterministic, void* stream) {
+  if (!ctx || numViews < 0 || (numViews > 0 && !views))
+    return fail(ctx, CR_ERR_INVALID, "cr_interpolate_views_backward: NULL argument");
+  return interpolateBackward(ctx, "cr_interpolate_views_backward", deterministic != 0, views, numViews, width, height,
+                             numChannels, stream);
 }
 
 cr_status cr_surface_resolve(const cr_surface* color, void* out, void* stream) {

@@ -320,6 +320,18 @@ __device__ __forceinline__ void stampStage(const Params& P, Stamp s) {
   if (threadIdx.x == 0) P.counters->stamp[s] = wall_clock64();
 }
 
+// Inclusive sum over the wave's lanes in DPP adds (shifts inside rows of 16,
+// then the rows' last lanes broadcast): 6 dependent additions, no LDS pipe.
+__device__ __forceinline__ uint32_t waveScan(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);   // row_shr:1
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);   // row_shr:2
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);   // row_shr:4
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);   // row_shr:8
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);   // row_bcast:15
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);   // row_bcast:31
+  return v;
+}
+
 // Host-side launchers, one per stage file.
 void launchReset(const Params& P, hipStream_t stream);
 void launchFinish(const Params& P, Counters* host, hipStream_t stream);
@@ -359,9 +371,27 @@ struct InterpGeom {
   int32_t width, height;        // viewport = surface size
   int32_t texW;                 // texel pitch of the id surface (rounded width, one sample)
   int32_t numChannels;
-  int32_t numTris;
-  int64_t numVertices;
 };
+// One view of a call: its inputs and outputs (forward: ids, out, triImage;
+// backward: triImage, gradOut, gradPos, gradAttr, acc).
+struct InterpView {
+  const uint32_t* ids;
+  const float* pos;
+  const float* attr;
+  const int32_t* tris;
+  float* out;
+  int32_t* triImage;
+  const float* gradOut;
+  float* gradPos;
+  float* gradAttr;
+  unsigned long long* acc;
+  int64_t numVertices;
+  int32_t numTris;
+  int32_t vec4;                 // set by the launcher: channels move as float4
+};
+// Views per launch: the views travel in the kernel's arguments (3 KB of the
+// 4 KB they may hold), so that a call needs no table in device memory.
+constexpr int kInterpViews = 32;
 // Box MSAA resolve of an RGBA8 surface into width x height pixels.
 void launchResolve(const uint32_t* tex, int32_t textureW, int32_t width, int32_t height, int32_t samplesLog2,
                    uint32_t* out, hipStream_t stream);
@@ -369,15 +399,12 @@ void launchResolve(const uint32_t* tex, int32_t textureW, int32_t width, int32_t
 // model position into the first 16 bytes of each outStride-byte record.
 void launchVertexPassthrough(const float* modelPos, int64_t numVertices, const float posToClip[16], void* out,
                              int64_t outStride, hipStream_t stream);
-void launchInterpForward(const InterpGeom& G, const uint32_t* ids, const float* pos, const float* attr,
-                         const int32_t* tris, float* out, int32_t* triImage, hipStream_t stream);
+void launchInterpForward(const InterpGeom& G, const InterpView* views, int numViews, hipStream_t stream);
 // gradPos (4 per vertex) and gradAttr (C per vertex) are overwritten.  The
-// per-(tile, triangle) FP64 sums are added with FP32 atomics (acc null), or,
-// bit-reproducibly, as 128-bit fixed-point integers in acc (2 * (4 + C) * V
-// 64-bit words) rounded to FP32 at the end.
-void launchInterpBackward(const InterpGeom& G, const int32_t* triImage, const float* pos, const float* attr,
-                          const int32_t* tris, const float* gradOut, float* gradPos, float* gradAttr,
-                          unsigned long long* acc, hipStream_t stream);
+// per-(tile, triangle) FP64 sums are added with FP32 atomics (acc null in
+// every view), or, bit-reproducibly, as 128-bit fixed-point integers in each
+// view's acc (2 * (4 + C) * V 64-bit words) rounded to FP32 at the end.
+void launchInterpBackward(const InterpGeom& G, const InterpView* views, int numViews, hipStream_t stream);
 
 // Largest v with start[v] <= b: the view owning workgroup (or group) b.
 // start has numViews + 1 nondecreasing entries; views without work have

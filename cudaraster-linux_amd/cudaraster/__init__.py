@@ -52,6 +52,7 @@ EXPORTS = [
     "cr_interpolate", "cr_interpolate_backward", "cr_batch_configure", "cr_vertex_shader_passthrough",
     "cr_surface_resolve", "cr_draw_triangles_noalloc", "cr_get_profile_counters", "cr_set_shader_constants",
     "cr_interpolate_ids", "cr_interpolate_backward_deterministic",
+    "cr_interpolate_views", "cr_interpolate_views_backward",
 ]
 
 
@@ -187,6 +188,8 @@ def load(path: str | None = None):
         "cr_set_shader_constants": [vp, ctypes.POINTER(ShaderConstants)],
         "cr_interpolate_ids": [vp, vp, i32, i32, vp, i64, vp, i32, vp, i32, vp, vp],
         "cr_interpolate_backward_deterministic": [vp, vp, i32, i32, vp, i64, vp, i32, vp, i32, vp, vp, vp, vp],
+        "cr_interpolate_views": [vp, vp, i32, i32, vp],
+        "cr_interpolate_views_backward": [vp, vp, i32, i32, i32, i32, i32, vp],
     }
     for name, args in sig.items():
         f = getattr(L, name)

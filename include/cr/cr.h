@@ -430,15 +430,15 @@ cr_status cr_interpolate_ids(cr_context* ctx, const int32_t* tri_image, int32_t 
                              const int32_t* tris, int32_t num_tris, float* out, void* stream);
 /* Backward: overwrites grad_pos[V][4] (z component 0) and grad_attr[V][C]
  * with dL/dpos and dL/dattr given grad_out[y][x][c] = dL/dout.  The terms
- * of each triangle's pixels within a 16x16 tile are summed in FP64 and added
- * to the outputs with FP32 atomics (summation order varies between runs in
- * the last bits).  Uses no context scratch. */
+ * of each vertex within a 16x16 tile are summed in FP64 and added to the
+ * outputs with FP32 atomics (summation order varies between runs in the last
+ * bits).  Uses no context scratch. */
 cr_status cr_interpolate_backward(cr_context* ctx, const int32_t* tri_image, int32_t width, int32_t height,
                                   const float* pos, int64_t num_vertices, const float* attr,
                                   int32_t num_channels, const int32_t* tris, int32_t num_tris,
                                   const float* grad_out, float* grad_pos, float* grad_attr, void* stream);
 /* The same gradients, bit-reproducible from run to run: each (tile,
- * triangle) FP64 sum is converted to a 128-bit fixed-point integer (2^-64
+ * vertex) FP64 sum, added up in a fixed order, is converted to a 128-bit fixed-point integer (2^-64
  * resolution; sums must stay below 2^63 in magnitude) and accumulated with
  * integer atomics, whose total does not depend on their order, then rounded
  * to FP32 once.  Uses a context scratch buffer of 16 bytes per output value
@@ -448,6 +448,30 @@ cr_status cr_interpolate_backward_deterministic(cr_context* ctx, const int32_t* 
                                                 const float* attr, int32_t num_channels, const int32_t* tris,
                                                 int32_t num_tris, const float* grad_out, float* grad_pos,
                                                 float* grad_attr, void* stream);
+/* Several views of one resolution and channel count in one launch per kernel:
+ * what the calls above do for each view in turn.  A view that needs no
+ * tri_image in the forward call passes NULL.  The forward call reads tri_id,
+ * pos, attr and tris and writes out and tri_image; the backward call reads
+ * tri_image, pos, attr, tris and grad_out and writes grad_pos and grad_attr.
+ * deterministic: as cr_interpolate_backward_deterministic. */
+typedef struct cr_interp_view {
+    const cr_surface* tri_id;
+    const float* pos;
+    int64_t num_vertices;
+    const float* attr;
+    const int32_t* tris;
+    int64_t num_tris;
+    float* out;
+    int32_t* tri_image;
+    const float* grad_out;
+    float* grad_pos;
+    float* grad_attr;
+} cr_interp_view;
+cr_status cr_interpolate_views(cr_context* ctx, const cr_interp_view* views, int32_t num_views,
+                               int32_t num_channels, void* stream);
+cr_status cr_interpolate_views_backward(cr_context* ctx, const cr_interp_view* views, int32_t num_views,
+                                        int32_t width, int32_t height, int32_t num_channels,
+                                        int32_t deterministic, void* stream);
 
 /* Passthrough vertex shader, the step before drawTriangles: replaces
  * vertexShader_passthrough (test/shader/PassThrough.cu:16-35) as the demo
