@@ -52,6 +52,7 @@ struct Tables {
     int ofs = 0, orderOfs = 0; // prefix (n + 1 entries) and order (n entries) in `starts`
   };
   int n = 0;
+  std::vector<int> members;    // the views, in the order of `params`
   Stage setup, coarse;
   std::vector<Stage> fine;
   DevBuf params, starts;
@@ -81,6 +82,7 @@ struct cr_batch {
   int banded = 0;                     // fine tile groups in XCD bands (1) or round-robin (0)
   int coarseThreads = 256;            // coarse workgroup size
   bool haveCounts = false;            // hostCounters hold every view's demand from a complete draw
+  bool moved = false;                 // views' buffers changed since the tables were built
   bool laidOut = false, useGraph = true, graphValid = false, tuned = false;
   hipStream_t capStream = nullptr;
   hipGraph_t graph = nullptr;
@@ -260,6 +262,7 @@ cr_status buildTables(cr_batch* b, Tables& T, const std::vector<int>& idx) {
   if (n > 0) CR_HIP(ctx, hipMemcpy(T.params.ptr, ps.data(), (size_t)n * sizeof(Params), hipMemcpyHostToDevice));
   CR_HIP(ctx, hipMemcpy(T.starts.ptr, st.data(), st.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   T.n = n;
+  T.members = idx;
   return CR_OK;
 }
 
@@ -360,6 +363,29 @@ cr_status clearCounters(cr_batch* b, hipStream_t stream) {
   return CR_OK;
 }
 
+// Writes the views' current vertex and index buffers into the tables of
+// views.  (In a small kernel on the draw's stream, the pointers in its
+// arguments: the captured graph stays as it is, and nothing is copied.)
+cr_status patchBuffers(cr_batch* b, hipStream_t stream) {
+  if (!b->moved) return CR_OK;
+  for (int g = 0; g < b->numGroups; g++) {
+    const Tables& T = b->groups[g];
+    for (int first = 0; first < T.n; first += kPatchViews) {
+      PatchTable P = {};
+      const int n = std::min(T.n - first, kPatchViews);
+      for (int k = 0; k < n; k++) {
+        const cr_view& d = b->views[T.members[first + k]].desc;
+        P.vertices[k] = static_cast<const uint8_t*>(d.vertices);
+        P.indices[k] = static_cast<const int32_t*>(d.indices);
+      }
+      launchPatchBatch(T.params.as<Params>(), P, first, n, stream);
+    }
+  }
+  CR_HIP(b->ctx, hipGetLastError());
+  b->moved = false;
+  return CR_OK;
+}
+
 // Grows the capacities of every view whose counters overflowed and re-draws
 // those views (only) until none does.
 cr_status settleOverflow(cr_batch* b, hipStream_t stream) {
@@ -406,7 +432,8 @@ cr_status drawBatch(cr_batch* b, hipStream_t stream, bool graph) {
     st = capture(b);
     if (st != CR_OK) return st;
   }
-  st = clearCounters(b, stream);
+  st = patchBuffers(b, stream);
+  if (st == CR_OK) st = clearCounters(b, stream);
   if (st != CR_OK) return st;
   b->countersClean = false;
   if (graph) {
@@ -660,6 +687,27 @@ cr_status cr_batch_reserve(cr_batch* b, int32_t view, int64_t maxSubtris, int64_
   v.maxTile = maxTile;
   b->laidOut = false;
   b->graphValid = false;
+  return CR_OK;
+}
+
+cr_status cr_batch_set_buffers(cr_batch* b, const void* const* vertices, const void* const* indices,
+                               int32_t numViews) {
+  if (!b || (numViews > 0 && (!vertices || !indices)))
+    return fail(b ? b->ctx : nullptr, CR_ERR_INVALID, "cr_batch_set_buffers: NULL argument");
+  if (numViews != (int32_t)b->views.size())
+    return fail(b->ctx, CR_ERR_INVALID, "cr_batch_set_buffers: %d views, the batch has %zu", numViews, b->views.size());
+  for (int i = 0; i < numViews; i++) {
+    cr_view v = b->views[i].desc;
+    v.vertices = vertices[i];
+    v.indices = indices[i];
+    const cr_status st = validateView(b->ctx, v, i);
+    if (st != CR_OK) return st;
+  }
+  for (int i = 0; i < numViews; i++) {
+    b->views[i].desc.vertices = vertices[i];
+    b->views[i].desc.indices = indices[i];
+  }
+  b->moved = true;
   return CR_OK;
 }
 

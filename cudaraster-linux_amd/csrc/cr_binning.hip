@@ -731,6 +731,18 @@ void launchCoarse(const Params& P, hipStream_t stream) {
     hipLaunchKernelGGL(coarseKernel<256>, dim3(((P.numBins + 7) >> 3) * 8), dim3(256), 0, stream, P);
 }
 
+// Points views [first, first + n) at other vertex and index buffers.
+__global__ void __launch_bounds__(kPatchViews) patchBatchKernel(Params* views, const PatchTable T, int first, int n) {
+  const int k = (int)threadIdx.x;
+  if (k >= n) return;
+  views[first + k].vertices = T.vertices[k];
+  views[first + k].indices = T.indices[k];
+}
+
+void launchPatchBatch(Params* views, const PatchTable& T, int first, int n, hipStream_t stream) {
+  hipLaunchKernelGGL(patchBatchKernel, dim3(1), dim3(kPatchViews), 0, stream, views, T, first, n);
+}
+
 void launchResetBatch(const Params* views, int numViews, hipStream_t stream) {
   if (numViews <= 0) return;
   hipLaunchKernelGGL(resetBatchKernel, dim3(numViews), dim3(64), 0, stream, views);

@@ -346,6 +346,13 @@ constexpr int kSetupChunkTris = 1024;
 // its own order: the k-th listed view is views[order[k]] and owns the
 // workgroups [blockStart[k], blockStart[k+1]).
 void launchResetBatch(const Params* views, int numViews, hipStream_t stream);
+// Vertex and index buffers of up to kPatchViews views, in kernel arguments.
+constexpr int kPatchViews = 128;
+struct PatchTable {
+  const uint8_t* vertices[kPatchViews];
+  const int32_t* indices[kPatchViews];
+};
+void launchPatchBatch(Params* views, const PatchTable& T, int first, int n, hipStream_t stream);
 // devBase, hostBase: the batch's counter blocks and their host copies.
 void launchFinishBatch(const Params* views, int numViews, const Counters* devBase, Counters* hostBase,
                        hipStream_t stream);

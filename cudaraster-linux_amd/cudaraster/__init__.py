@@ -52,7 +52,7 @@ EXPORTS = [
     "cr_interpolate", "cr_interpolate_backward", "cr_batch_configure", "cr_vertex_shader_passthrough",
     "cr_surface_resolve", "cr_draw_triangles_noalloc", "cr_get_profile_counters", "cr_set_shader_constants",
     "cr_interpolate_ids", "cr_interpolate_backward_deterministic",
-    "cr_interpolate_views", "cr_interpolate_views_backward",
+    "cr_interpolate_views", "cr_interpolate_views_backward", "cr_batch_set_buffers",
 ]
 
 
@@ -188,6 +188,7 @@ def load(path: str | None = None):
         "cr_set_shader_constants": [vp, ctypes.POINTER(ShaderConstants)],
         "cr_interpolate_ids": [vp, vp, i32, i32, vp, i64, vp, i32, vp, i32, vp, vp],
         "cr_interpolate_backward_deterministic": [vp, vp, i32, i32, vp, i64, vp, i32, vp, i32, vp, vp, vp, vp],
+        "cr_batch_set_buffers": [vp, vp, vp, i32],
         "cr_interpolate_views": [vp, vp, i32, i32, vp],
         "cr_interpolate_views_backward": [vp, vp, i32, i32, i32, i32, i32, vp],
     }
@@ -561,6 +562,13 @@ class Batch:
     def reserve(self, view, max_subtris, max_bin_entries, max_tile_entries):
         _check(load().cr_batch_reserve(self._h, int(view), int(max_subtris), int(max_bin_entries),
                                        int(max_tile_entries)), self._raster.ctx)
+
+    def set_buffers(self, vertices, indices):
+        """Other vertex and index buffers of the same counts for the views
+        (lists of raw device pointers), from the next draw on."""
+        n = len(vertices)
+        v, i = (ctypes.c_void_p * n)(*vertices), (ctypes.c_void_p * n)(*indices)
+        _check(load().cr_batch_set_buffers(self._h, v, i, n), self._raster.ctx)
 
     def configure(self, fine_tiles_per_group=4, fine_banded=0, coarse_threads=256, view_groups=1):
         c = (ctypes.c_int32 * 4)(fine_tiles_per_group, fine_banded, coarse_threads, view_groups)

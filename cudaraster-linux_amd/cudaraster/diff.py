@@ -11,7 +11,7 @@ passes are HIP kernels in libcr.so.
 """
 from __future__ import annotations
 
-import ctypes
+import numpy as np
 
 from . import (CR_ERR_OVERFLOW, CR_OK, Batch, CrError, CudaRaster, CudaSurface, FORMAT_DEPTH32, FORMAT_RGBA8,
                FORMAT_TRIANGLE_ID, View, _check, load, pipe_desc, SHADER_CONSTANT, BLEND_REPLACE, RENDER_DEPTH)
@@ -78,28 +78,25 @@ class InterpolateViews:
                 H, W, C = raster.height, raster.width, attr[0].shape[1]
                 out = torch.empty((n, H, W, C), dtype=torch.float32, device=pos[0].device)
                 ids = torch.empty((n, H, W), dtype=torch.int32, device=pos[0].device)
-                # Visibility of every view in one batched draw, then each
-                # view's interpolation from its own triangle-id surface.
+                raster._check_views(pos, attr, tris, ids, C)
+                # Visibility of every view in one batched draw, then the
+                # views' interpolation from their triangle-id surfaces.
                 surfaces = raster._draw_views(pos, tris)
-                for i in range(n):
-                    raster._interpolate(pos[i].detach(), attr[i].detach(), tris[i], out[i], ids[i],
-                                        surface=surfaces[i])
+                raster._interpolate_views(pos, attr, tris, out, ids, surfaces)
                 ctx.save_for_backward(ids, *tensors)
                 ctx.raster, ctx.n = raster, n
                 ctx.mark_non_differentiable(ids)
+                ctx.set_materialize_grads(False)
                 return out, ids
 
             @staticmethod
             def backward(ctx, grad_out, _grad_ids):
                 n = ctx.n
+                if grad_out is None:
+                    return (None,) * (2 + 3 * n)
                 ids, *tensors = ctx.saved_tensors
                 pos, attr, tris = tensors[:n], tensors[n:2 * n], tensors[2 * n:3 * n]
-                grad_out = grad_out.contiguous()
-                gp, ga = [], []
-                for i in range(n):
-                    a, b = ctx.raster._interpolate_backward(pos[i], attr[i], tris[i], ids[i], grad_out[i])
-                    gp.append(a)
-                    ga.append(b)
+                gp, ga = ctx.raster._interpolate_views_backward(pos, attr, tris, ids, grad_out.contiguous())
                 return (None, None, *gp, *ga, *([None] * n))
 
         cls._fn = _InterpolateViews
@@ -126,38 +123,33 @@ class DiffRasterizer:
         # Positions only (16-byte vertices), depth test on, constant colour.
         self.cr.setPixelPipe(pipe_desc(16, SHADER_CONSTANT, BLEND_REPLACE, 0, RENDER_DEPTH))
         # render_views: the batched visibility draw of the last view sizes
-        # (signature, cr_batch, per-view surfaces, staging buffers).
+        # (signature, cr_batch, per-view surfaces).
         self._views = None
 
     def _draw_views(self, pos, tris):
         """Exact visibility of several views in one batched draw (cr_batch:
         one launch per stage over all views, the same images as drawing them
-        in turn); returns each view's triangle-id surface.  The batch, its
-        per-view surfaces and staging buffers for the positions and indices
+        in turn) straight from the caller's positions and indices; returns
+        each view's triangle-id surface.  The batch and its per-view surfaces
         are kept for the next call with the same view sizes."""
         import torch
-        for p, t in zip(pos, tris):
-            if not (p.is_cuda and p.dtype == torch.float32 and p.dim() == 2 and p.shape[1] == 4):
-                raise CrError(1, "pos must be a float32 [V, 4] device tensor")
-            if not (t.is_cuda and t.dtype == torch.int32 and t.dim() == 2 and t.shape[1] == 3):
-                raise CrError(1, "tris must be an int32 [T, 3] device tensor")
         key = tuple((int(p.shape[0]), int(t.shape[0]), p.device.index) for p, t in zip(pos, tris))
+        vertices = [p.data_ptr() if k[0] else None for p, k in zip(pos, key)]
+        indices = [t.data_ptr() if k[1] else None for t, k in zip(tris, key)]
         if self._views is None or self._views[0] != key:
             self._close_views()
-            vbuf = [torch.empty((k[0], 4), dtype=torch.float32, device=p.device) for k, p in zip(key, pos)]
-            ibuf = [torch.empty((k[1], 3), dtype=torch.int32, device=p.device) for k, p in zip(key, pos)]
             surfaces, views = [], []
             pipe = pipe_desc(16, SHADER_CONSTANT, BLEND_REPLACE, 0, RENDER_DEPTH)
             try:
-                for vb, ib in zip(vbuf, ibuf):
+                for k, vp, ip in zip(key, vertices, indices):
                     trio = (CudaSurface((self.width, self.height), FORMAT_RGBA8, 1),
                             CudaSurface((self.width, self.height), FORMAT_DEPTH32, 1),
                             CudaSurface((self.width, self.height), FORMAT_TRIANGLE_ID, 1))
                     surfaces.append(trio)
                     v = View()
                     v.color, v.depth, v.tri_id = (s.handle.value for s in trio)
-                    v.vertices, v.num_vertices = (vb.data_ptr() if vb.numel() else None), vb.shape[0]
-                    v.indices, v.num_tris = (ib.data_ptr() if ib.numel() else None), ib.shape[0]
+                    v.vertices, v.num_vertices = vp, k[0]
+                    v.indices, v.num_tris = ip, k[1]
                     v.deferred_clear = 1
                     v.pipe = pipe
                     v.clear_color[:] = [0.0, 0.0, 0.0, 0.0]
@@ -169,17 +161,15 @@ class DiffRasterizer:
                     for sf in trio:
                         sf.close()
                 raise
-            self._views = (key, batch, surfaces, vbuf, ibuf)
-        _, batch, surfaces, vbuf, ibuf = self._views
-        for vb, ib, p, t in zip(vbuf, ibuf, pos, tris):
-            vb.copy_(p.detach())
-            ib.copy_(t)
+            self._views = (key, batch, surfaces)
+        _, batch, surfaces = self._views
+        batch.set_buffers(vertices, indices)
         batch.draw(torch.cuda.current_stream())
         return [trio[2] for trio in surfaces]
 
     def _close_views(self):
         if self._views is not None:
-            _, batch, surfaces, _, _ = self._views
+            _, batch, surfaces = self._views
             self._views = None
             batch.close()
             for trio in surfaces:
@@ -262,16 +252,15 @@ class DiffRasterizer:
                 tuple(tri_image.shape) == (self.height, self.width)):
             raise CrError(1, "tri_image must be a contiguous int32 [H, W] device tensor at the rasterizer's resolution")
 
-    def _interpolate(self, pos, attr, tris, out, tri_image, channels=None, surface=None):
-        """Interpolates from the triangle ids of `surface` (default: this
-        rasterizer's own, from the last _draw) and copies them to tri_image."""
+    def _interpolate(self, pos, attr, tris, out, tri_image, channels=None):
+        """Interpolates from the triangle ids of this rasterizer's last _draw
+        and copies them to tri_image."""
         C = attr.shape[1] if channels is None else channels
         self._check_inputs(pos, attr, tris, tri_image, C)
         hw = self.height * self.width
         if C > 0 and (out.numel() != hw * C or not out.is_contiguous() or not out.is_cuda):
             raise CrError(1, "interpolation output buffers do not match the rasterizer's resolution")
-        ids = self.ids if surface is None else surface
-        _check(load().cr_interpolate(self.cr.ctx, ids.handle, pos.data_ptr(), pos.shape[0],
+        _check(load().cr_interpolate(self.cr.ctx, self.ids.handle, pos.data_ptr(), pos.shape[0],
                                      attr.data_ptr() if attr is not None else None, C, tris.data_ptr(),
                                      tris.shape[0], out.data_ptr(), tri_image.data_ptr(), _stream()), self.cr.ctx)
 
@@ -283,6 +272,59 @@ class DiffRasterizer:
         _check(load().cr_interpolate_ids(self.cr.ctx, tri_image.data_ptr(), self.width, self.height, pos.data_ptr(),
                                          pos.shape[0], attr.data_ptr(), C, tris.data_ptr(), tris.shape[0],
                                          out.data_ptr(), _stream()), self.cr.ctx)
+
+    def _check_views(self, pos, attr, tris, ids, channels):
+        """_check_inputs for several views at once."""
+        import torch
+        f32, i32, n = torch.float32, torch.int32, len(pos)
+        for p, a, t in zip(pos, attr, tris):
+            ps, ts = p.shape, t.shape
+            if not (p.is_cuda and p.dtype == f32 and len(ps) == 2 and ps[1] == 4 and p.is_contiguous()):
+                raise CrError(1, "pos must be a contiguous float32 [V, 4] device tensor")
+            if p.data_ptr() & 15:
+                raise CrError(1, "pos must be 16-byte aligned")
+            if not (t.is_cuda and t.dtype == i32 and len(ts) == 2 and ts[1] == 3 and t.is_contiguous()):
+                raise CrError(1, "tris must be a contiguous int32 [T, 3] device tensor")
+            if channels > 0 and not (a.is_cuda and a.dtype == f32 and a.shape == (ps[0], channels) and
+                                     a.is_contiguous()):
+                raise CrError(1, "attr must be a contiguous float32 [V, C] device tensor with one row per vertex")
+        if not (ids.is_cuda and ids.dtype == i32 and ids.is_contiguous() and
+                ids.shape == (n, self.height, self.width)):
+            raise CrError(1, "the id images must be one contiguous int32 [n, H, W] device tensor")
+
+    def _view_table(self, pos, attr, tris, ids):
+        """cr_interp_view records (eleven 8-byte words each) with the inputs
+        and the id images filled in, as an int64 array."""
+        t = np.array([(0, p.data_ptr(), p.shape[0], a.data_ptr(), r.data_ptr(), r.shape[0], 0, 0, 0, 0, 0)
+                      for p, a, r in zip(pos, attr, tris)], dtype=np.int64)
+        t[:, 7] = ids.data_ptr() + np.arange(len(pos)) * (self.height * self.width * 4)
+        return t
+
+    def _interpolate_views(self, pos, attr, tris, out, ids, surfaces):
+        """The views' interpolation from `surfaces` into out [n, H, W, C],
+        their triangle ids into ids [n, H, W]; checked by _check_views."""
+        t = self._view_table(pos, attr, tris, ids)
+        t[:, 0] = [s.handle.value for s in surfaces]
+        t[:, 6] = out.data_ptr() + np.arange(len(pos)) * (self.height * self.width * out.shape[3] * 4)
+        _check(load().cr_interpolate_views(self.cr.ctx, t.ctypes.data, len(pos), out.shape[3], _stream()),
+               self.cr.ctx)
+
+    def _interpolate_views_backward(self, pos, attr, tris, ids, grad_out):
+        import torch
+        n, C = len(pos), attr[0].shape[1]
+        self._check_views(pos, attr, tris, ids, C)
+        if (grad_out.dtype != torch.float32 or grad_out.numel() != ids.numel() * C or
+                not grad_out.is_contiguous()):
+            raise CrError(1, "gradient of the image does not match its shape")
+        gp = [torch.empty_like(p) for p in pos]
+        ga = [torch.empty_like(a) for a in attr]
+        t = self._view_table(pos, attr, tris, ids)
+        t[:, 8] = grad_out.data_ptr() + np.arange(n) * (self.height * self.width * C * 4)
+        t[:, 9] = [x.data_ptr() for x in gp]
+        t[:, 10] = [x.data_ptr() for x in ga]
+        _check(load().cr_interpolate_views_backward(self.cr.ctx, t.ctypes.data, n, self.width, self.height, C,
+                                                    1 if self.deterministic else 0, _stream()), self.cr.ctx)
+        return gp, ga
 
     def _interpolate_backward(self, pos, attr, tris, tri_image, grad_out):
         import torch

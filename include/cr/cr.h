@@ -381,6 +381,12 @@ cr_status cr_batch_autotune(cr_batch* batch, void* stream);
  * draw then grows them. */
 cr_status cr_batch_reserve(cr_batch* batch, int32_t view, int64_t max_subtris, int64_t max_bin_entries,
                            int64_t max_tile_entries);
+/* Other vertex and index buffers for the batch's views, of the same vertex and
+ * triangle counts, from the next draw on (arrays of num_views pointers; the
+ * conditions of cr_batch_create).  The buffers are read by later draws only
+ * while those run. */
+cr_status cr_batch_set_buffers(cr_batch* batch, const void* const* vertices, const void* const* indices,
+                               int32_t num_views);
 /* 0: launch the stages directly on each draw instead of replaying a graph. */
 cr_status cr_batch_use_graph(cr_batch* batch, int32_t enable);
 /* Sets the launch configuration the autotuner otherwise chooses (images do
