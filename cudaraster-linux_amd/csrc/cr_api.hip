@@ -79,6 +79,12 @@ void clearValues(const float rgba[4], float depth, uint32_t* color, uint32_t* en
   *encodedDepth = encodeDepth((uint32_t)std::min<uint64_t>(q, 0xFFFFFFFFull));
 }
 
+double clockTick(int device) {
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || khz <= 0) khz = 100000;
+  return 1e-3 / khz;
+}
+
 cr_status validatePipe(cr_context* ctx, const cr_pipe_desc* p) {
   if (p->samples_log2 < 0 || p->samples_log2 > 3) return fail(ctx, CR_ERR_INVALID, "pipe: samples_log2 must be 0..3");
   if (p->vertex_struct_size < 16 || (p->vertex_struct_size & 15))
@@ -371,9 +377,6 @@ cr_status cr_context_create(cr_context** out) {
   if (e == hipSuccess)
     e = hipHostMalloc((void**)&ctx->hostProf, 2 * kProfCount * sizeof(unsigned long long), hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&ctx->hostCountersDev, ctx->hostCounters, 0);
-  int khz = 0;
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device);
-  if (khz > 0) ctx->clockSeconds = 1e-3 / khz;
   if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->evPending, hipEventDisableTiming);
   if (e != hipSuccess) {
     cr_context_destroy(ctx);
@@ -617,8 +620,9 @@ cr_status cr_get_stats(cr_context* ctx, cr_stats* out) {
   // setup kernel: its time is part of setup_time and bin_time is 0.  (A draw
   // without triangles has no setup stage and no setup stamp.)
   const uint64_t* s = ctx->hostCounters->stamp;
+  const double tick = clockTick(ctx->device);
   auto seconds = [&](uint64_t from, uint64_t to) {
-    return from != 0 && to > from ? (float)((double)(to - from) * ctx->clockSeconds) : 0.0f;
+    return from != 0 && to > from ? (float)((double)(to - from) * tick) : 0.0f;
   };
   out->setup_time = seconds(s[kStampSetup], s[kStampCoarse]);
   out->bin_time = 0.0f;

@@ -87,7 +87,8 @@ struct cr_batch {
   hipStream_t capStream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  float lastMs = 0.0f, tunedMs = 0.0f;
+  uint64_t lastTicks = 0;             // GPU time of the last draw, in wall clock ticks
+  float tunedMs = 0.0f;
   int64_t retries = 0;
   size_t reserved = 0;
 };
@@ -452,7 +453,7 @@ cr_status drawBatch(cr_batch* b, hipStream_t stream, bool graph) {
       if (s[k] != 0) first = std::min(first, s[k]);
     last = std::max(last, s[kStampEnd]);
   }
-  b->lastMs = last > first ? (float)((double)(last - first) * ctx->clockSeconds * 1e3) : 0.0f;
+  b->lastTicks = last > first ? last - first : 0;
   return settleOverflow(b, stream);
 }
 
@@ -611,6 +612,7 @@ cr_status cr_batch_autotune(cr_batch* b, void* stream_) {
   //    list views longest-first by the measured entries per bin and tile).
   int bestW = b->tilesPerGroup, bestBanded = b->banded, bestCoarse = b->coarseThreads;
   float bestMs = 1e30f;
+  const double tick = clockTick(b->device) * 1e3;
   for (int banded = 0; banded < 2; banded++) {
     for (int trial = 0; trial < 3 + 1; trial++) {
       // three fine shapes with the current coarse size, then the other
@@ -626,7 +628,7 @@ cr_status cr_batch_autotune(cr_batch* b, void* stream_) {
         st = saveSurfaces(b, stream, true);
         if (st == CR_OK) st = drawBatch(b, stream, false);
         if (st != CR_OK) return st;
-        if (rep > 0) ms[rep - 1] = b->lastMs;
+        if (rep > 0) ms[rep - 1] = (float)((double)b->lastTicks * tick);
       }
       std::sort(ms, ms + 3);
       if (ms[1] < bestMs) {
@@ -654,7 +656,7 @@ cr_status cr_batch_autotune(cr_batch* b, void* stream_) {
       st = saveSurfaces(b, stream, true);
       if (st == CR_OK) st = drawBatch(b, stream, false);
       if (st != CR_OK) return st;
-      if (rep > 0) ms[rep - 1] = b->lastMs;
+      if (rep > 0) ms[rep - 1] = (float)((double)b->lastTicks * tick);
     }
     std::sort(ms, ms + 3);
     if (ms[1] < bestMs) {
@@ -744,7 +746,7 @@ cr_status cr_batch_get_info(const cr_batch* b, cr_batch_info* out) {
   out->tuned = b->tuned ? 1 : 0;
   out->retries = b->retries;
   out->reserved_bytes = (int64_t)b->reserved;
-  out->last_gpu_ms = b->lastMs;
+  out->last_gpu_ms = (float)((double)b->lastTicks * clockTick(b->device) * 1e3);
   out->tuned_gpu_ms = b->tunedMs;
   return CR_OK;
 }

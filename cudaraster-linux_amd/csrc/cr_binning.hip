@@ -692,7 +692,8 @@ __global__ void __launch_bounds__(CT) coarseBatchKernel(const Params* __restrict
                                                         const int32_t* __restrict__ blockStart,
                                                         const int32_t* __restrict__ order, int numViews) {
   const int k = findView(blockStart, numViews, (int)blockIdx.x);
-  coarseBody<CT>(views[order[k]], (int)blockIdx.x - blockStart[k]);
+  const Params P = loadParams(&views[order[k]]);
+  coarseBody<CT>(P, (int)blockIdx.x - blockStart[k]);
 }
 
 // One workgroup per view: clears the view's counter block.

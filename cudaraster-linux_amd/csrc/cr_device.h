@@ -315,6 +315,48 @@ __host__ __device__ inline int selectCentroid(int s, uint32_t mask) {
   return best;
 }
 
+// One view's parameters from a batch's table, by scalar loads into registers
+// of the caller (what it does not use is not loaded), with the pointers known
+// to be global: through a reference to the table every access would be a
+// generic one, which waits for the LDS counter too.
+template <class T>
+__device__ __forceinline__ void makeGlobal(T*& p) {
+  p = (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;
+}
+__device__ __forceinline__ Params loadParams(const Params* view) {
+  using Word = const __attribute__((address_space(4))) uint64_t;
+  static_assert(sizeof(Params) % 8 == 0 && alignof(Params) == 8, "whole words");
+  Word* w = (Word*)(uintptr_t)view;
+  Params P;
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(Params) / 8); i++) reinterpret_cast<uint64_t*>(&P)[i] = w[i];
+  makeGlobal(P.vertices);
+  makeGlobal(P.indices);
+  makeGlobal(P.tileFrags);
+  makeGlobal(P.chunkSubtris);
+  makeGlobal(P.prof);
+  makeGlobal(P.materials);
+  makeGlobal(P.triMaterial);
+  makeGlobal(P.atlas);
+  makeGlobal(P.triSubtris);
+  makeGlobal(P.triHeader);
+  makeGlobal(P.triData);
+  makeGlobal(P.subtriTri);
+  makeGlobal(P.chunkBase);
+  makeGlobal(P.binCnt);
+  makeGlobal(P.binOff);
+  makeGlobal(P.binList);
+  makeGlobal(P.tileStart);
+  makeGlobal(P.tileCount);
+  makeGlobal(P.tileList);
+  makeGlobal(P.tileSegNext);
+  makeGlobal(P.color);
+  makeGlobal(P.depth);
+  makeGlobal(P.triid);
+  makeGlobal(P.counters);
+  return P;
+}
+
 // Called by every thread of a stage's workgroup 0.
 __device__ __forceinline__ void stampStage(const Params& P, Stamp s) {
   if (threadIdx.x == 0) P.counters->stamp[s] = wall_clock64();

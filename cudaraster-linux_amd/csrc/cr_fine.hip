@@ -44,7 +44,11 @@ struct Rec {
   static constexpr int SLOT = ZS + N;          // subtriangle slot (deferred shading: slot << 4)
   static constexpr int TRI = SLOT + 1;         // source triangle index
   static constexpr int SH = TRI + 1;           // in-order shading: W/U/V planes (9) + colours (12)
-  static constexpr int SIZE_VIS = (SH + 3) & ~3;
+  static constexpr int M = SH;                 // deferred shading: largest threshold per edge [3]
+  // An odd multiple of 16 bytes: the lanes' records, up to 16 apart, start in
+  // different banks.
+  static constexpr int SIZE_VIS = ((M + 3 + 3) & ~7) + 4;
+  static_assert(SIZE_VIS >= M + 4 && SIZE_VIS % 8 == 4, "three thresholds and a spare last word");
   static constexpr int SIZE_FULL = (SH + 21 + 3) & ~3;
 };
 
@@ -152,7 +156,28 @@ __device__ __forceinline__ float4 varying0(const uint8_t* verts, uint32_t vi, in
   return *reinterpret_cast<const float4*>(verts + (uint64_t)vi * (uint32_t)stride + 16);
 }
 
+// Bit rows of each half-wave transposed: bit b of lane l becomes bit l of
+// lane b (l, b < 32, per half).  Five exchange steps; a lane keeps its own
+// half of the bits and takes the partner's other half, rotated into place.
+__device__ __forceinline__ uint32_t transposeBits(uint32_t x, int lane) {
+  auto step = [&](uint32_t y, uint32_t low, int sh) {
+    const bool up = (lane & sh) != 0;
+    const uint32_t keep = up ? ~low : low;
+    const uint32_t rot = __builtin_amdgcn_alignbit(y, y, up ? (uint32_t)sh : (uint32_t)(32 - sh));
+    x = (x & keep) | (rot & ~keep);
+  };
+  step((uint32_t)__builtin_amdgcn_ds_swizzle((int)x, 0x401F), 0x0000FFFFu, 16);              // lane ^ 16
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false), 0x00FF00FFu, 8);   // row_ror:8
+  step((uint32_t)__builtin_amdgcn_ds_swizzle((int)x, 0x101F), 0x0F0F0F0Fu, 4);               // lane ^ 4
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false), 0x33333333u, 2);    // quad_perm 2,3,0,1
+  step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false), 0x55555555u, 1);    // quad_perm 1,0,3,2
+  return x;
+}
+
 constexpr int kFineWaves = 4;     // tiles (waves) per workgroup
+// Batches of at most this many records walk every record over the whole
+// tile: the pixels' record masks cost as much as three or four steps.
+constexpr uint32_t kFewRecords = 4;
 constexpr int kChunk = 32;        // triangles set up per chunk
 constexpr int kMaxDefer = 8;      // chunks hierarchical-Z survivors may wait before their walk
 
@@ -208,7 +233,10 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
   const int32_t blend = BL >= 0 ? BL : P.blend;
 
   if (group == 0) stampStage(P, kStampFine);
-  const int lane = threadIdx.x & 63;
+  int lane = threadIdx.x & 63;
+  // (Opaque: what depends on the lane alone is not kept in registers over a
+  // batched workgroup's rounds.)
+  __asm__ volatile("" : "+v"(lane));
   // Wave-uniform, so the tile's coordinates and addresses are scalars.
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   uint32_t* rec = recAll + wave * (kChunk * RS);
@@ -243,11 +271,11 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
   uint32_t col[N], dep[N], aux[N];   // aux: VIS -> (slot << 4 | centroid) or ~0; else triangle id
   if (P.deferredClear) {
 #pragma unroll
-    for (int i = 0; i < N; i++) { col[i] = P.clearColor; dep[i] = P.clearDepth; aux[i] = 0xFFFFFFFFu; }
+    for (int i = 0; i < N; i++) { if (!VIS) col[i] = P.clearColor; dep[i] = P.clearDepth; aux[i] = 0xFFFFFFFFu; }
   } else {
 #pragma unroll
     for (int i = 0; i < N; i++) {
-      col[i] = color[texel + i * 8];
+      if (!VIS) col[i] = color[texel + i * 8];
       dep[i] = depth[texel + i * 8];
       aux[i] = VIS ? 0xFFFFFFFFu : (idOn ? triid[texel + i * 8] : 0xFFFFFFFFu);
     }
@@ -259,7 +287,6 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
   const int32_t lx16 = lx << kSubpixelLog2, ly16 = ly << kSubpixelLog2;
   const uint32_t lxN = (uint32_t)(lx * N), lyN = (uint32_t)(ly * N);
   const uint32_t pixN = lxN | (lyN << 16);
-  const uint32_t quadShift = (uint32_t)((((ly >> 2) << 1) | (lx >> 2)) * 8);   // byte of this lane's quadrant
   const uint32_t tileSx = (uint32_t)(tx * 8 * N), tileSy = (uint32_t)(ty * 8 * N);
   constexpr CentroidOrder<S> co;
 
@@ -374,9 +401,6 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
         const uint32_t nb = min((uint32_t)kChunk, total - b);
         uint32_t* r = rec + lane * RS;
         const bool su = lane < (int)nb;
-        // Deferred shading: the 4x4-pixel quadrants of the tile this record
-        // may cover (bit (ly >= 4) * 2 + (lx >= 4)).
-        uint32_t quads = 0;
         waveSync();                            // the queue stores (or the last walk's reads) are done
         if (su) {
           const uint32_t slot = r[b == 0 ? Q0 : Q1];
@@ -398,7 +422,6 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
           // sample's threshold, i.e. its largest value over the tile is at most
           // the smallest threshold.  Exactly the per-sample test's outcome.
           bool full = true;
-          if (VIS) quads = 15u;
 #pragma unroll
           for (int k = 0; k < 3; k++) {
             const int kn = (k + 1) % 3;
@@ -430,17 +453,7 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
               maxR = max(maxR, rk);
             }
             full = full && __mul24(112, max(dy, 0)) + __mul24(112, max(-dx, 0)) <= minR;
-            if (VIS) {
-              // A quadrant none of whose samples can pass this edge: the
-              // smallest L over its pixels (lx16 in 64*qx + {0..48}, ly16 in
-              // 64*qy + {0..48}) exceeds the largest threshold.  |d| < 2^17:
-              // every term below fits 25 bits.
-              const int32_t ndx = -dx;
-              const int32_t m00 = (dy < 0 ? __mul24(48, dy) : 0) + (ndx < 0 ? __mul24(48, ndx) : 0);
-              const int32_t ex = dy * 64, ey = ndx * 64;
-              quads &= (m00 <= maxR ? 1u : 0u) | (m00 + ex <= maxR ? 2u : 0u) | (m00 + ey <= maxR ? 4u : 0u) |
-                       (m00 + ex + ey <= maxR ? 8u : 0u);
-            }
+            if (VIS) r[L::M + k] = (uint32_t)maxR;
             r[L::D + 2 * k] = (uint32_t)dy;
             r[L::D + 2 * k + 1] = (uint32_t)(-dx);
           }
@@ -481,43 +494,70 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
             q[15] = __float_as_uint(c1.z); q[16] = __float_as_uint(c1.w); q[17] = __float_as_uint(c2.x);
             q[18] = __float_as_uint(c2.y); q[19] = __float_as_uint(c2.z); q[20] = __float_as_uint(c2.w);
           }
-          // Quadrant queue slots start empty (this record's queue entry was
-          // read above).
-          if (VIS) r[Q0] = 0xFFFFFFFFu;
         }
         waveSync();
 
-        // Deferred shading: per 4x4 quadrant, the batch's records that may
-        // cover it, in submission order -- byte q of record i's word Q0 is the
-        // index of quadrant q's i-th record (0xFF past its end).  Step i of the
-        // walk takes the i-th record of every quadrant, so the quadrants walk
-        // their own records side by side; their pixels are disjoint, so every
-        // pixel still sees its triangles in submission order, and a step
-        // serves up to four small triangles.
-        uint32_t steps = nb;
-        if (VIS) {
-          steps = 0;
+        // Deferred shading: per pixel, the batch's records that may cover it,
+        // as a bit mask.  Lanes l and l + 32 work out record l's pixels in
+        // rows 0-3 and 4-7 (a byte per row); transposing the bits within
+        // each half turns 32 records' pixels into 32 pixels' records, and
+        // lane p holds pixel p's.  Every pixel then walks its own records in
+        // submission order, so that a batch takes as many steps as its most
+        // covered pixel has records.
+        //
+        // The pixels of row y that can pass an edge are those with
+        // 16 x dy + 16 y (-dx) <= maxR (at the sample with the largest
+        // threshold): x below (dy >= 0) or from (dy < 0) the cut
+        // (maxR - 16 y (-dx)) / (16 dy).  In floats, with a margin for their
+        // rounding that only ever admits a pixel too many (the walk tests
+        // every sample exactly); dy = 0 acts as a tiny positive one.
+        //
+        // What bounds the stage is VALU issue; a batch of 30 records of the
+        // 1M-triangle workload takes 10 such steps, where one queue per 4x4
+        // quadrant took 15 (and a record for the whole wave 30): fine
+        // 180 -> 157 us there, a 512x512 1x batch 216 -> 165 us, a batch of
+        // small views with deep lists 104 + 67 -> 73 + 52 us.
+        uint32_t mine = 0;
+        if (VIS && nb <= kFewRecords) {
+          mine = (1u << nb) - 1u;
+        } else if (VIS) {
+          const uint32_t* r = rec + (lane & 31) * RS;
+          const float row0 = lane >= 32 ? 4.0f : 0.0f;
+          float cut[3], st[3];
+          uint32_t side[3];
 #pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const uint64_t m = __ballot((quads >> q) & 1u);
-            steps = max(steps, (uint32_t)__popcll(m));
-            if ((quads >> q) & 1u)
-              reinterpret_cast<uint8_t*>(rec + rankBelow(m) * RS + Q0)[q] = (uint8_t)lane;
+          for (int k = 0; k < 3; k++) {
+            const int32_t dy = (int32_t)r[L::D + 2 * k], ndx = (int32_t)r[L::D + 2 * k + 1];
+            const float rcp = dy != 0 ? __builtin_amdgcn_rcpf((float)(16 * dy)) : 1e20f;
+            const float at = ((float)(int32_t)r[L::M + k] + 0.5f) * rcp;
+            st[k] = (float)(-16 * ndx) * rcp;
+            const float margin = fmaf(fmaf(fabsf(st[k]), 8.0f, fabsf(at)), 0x1p-20f, 0x1p-10f);
+            cut[k] = fmaf(row0, st[k], at) + 1.0f + (dy < 0 ? -margin : margin);
+            side[k] = dy < 0 ? 0xFFu : 0u;
           }
-          waveSync();
+#pragma unroll
+          for (int y = 0; y < 4; y++) {
+            uint32_t m = 0xFFu;
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+              const float c = __builtin_amdgcn_fmed3f(fmaf((float)y, st[k], cut[k]), 0.0f, 8.0f);
+              m &= ((1u << (uint32_t)c) - 1u) ^ side[k];
+            }
+            mine |= m << (8 * y);
+          }
+          if ((lane & 31) >= (int)nb) mine = 0;
+          mine = transposeBits(mine, lane);
         }
 
         // ---- walk the batch's triangles in submission order --------------------
-        for (uint32_t j = 0; j < steps; j++) {
+        for (uint32_t j = 0; VIS ? mine != 0 : j < nb; j++) {
           // In-order shading: record j for the whole wave (uniform address).
-          // Deferred shading: this lane's quadrant's j-th record; lanes whose
-          // quadrant has no j-th record read record 31 and take no part.
-          uint64_t validM = ~0ull;
+          // Deferred shading: this lane's next record; lanes without one are
+          // done (and not in the ballots below).
           const uint32_t* r = rec + j * RS;
           if (VIS) {
-            const uint32_t t = (r[Q0] >> quadShift) & 0xFFu;
-            validM = __ballot(t < (uint32_t)kChunk);
-            r = rec + min(t, (uint32_t)kChunk - 1) * RS;
+            r = rec + (uint32_t)__builtin_ctz(mine) * RS;
+            mine &= mine - 1u;
           }
           const uint32_t* cur = r;
           // |lx16|,|ly16| < 2^7 and |d| < 2^17: 24-bit multiplies are exact.
@@ -542,7 +582,7 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
 #pragma unroll
             for (int i = 0; i < N; i++) {
               covM[i] = __ballot(Lk[0] <= (int32_t)cur[L::R + i]) & __ballot(Lk[1] <= (int32_t)cur[L::R + N + i]) &
-                        __ballot(Lk[2] <= (int32_t)cur[L::R + 2 * N + i]) & validM;
+                        __ballot(Lk[2] <= (int32_t)cur[L::R + 2 * N + i]);
               anyM |= covM[i];
             }
           }
@@ -646,18 +686,27 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
 
   // The pixel's coordinates and surface offset, derived again from the lane
   // index (v_mbcnt) instead of being held in registers through the walk.
-  const int laneE = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  int laneE = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  __asm__ volatile("" : "+v"(laneE));
   const int pxE = (tx << kTileLog2) + (laneE & 7), pyE = (ty << kTileLog2) + (laneE >> 3);
-  const size_t texelE = (size_t)pyE * pitch + (size_t)tx * (8 * N) + (laneE & 7);
+  const size_t tileRowE = (size_t)pyE * pitch + (size_t)tx * (8 * N);
 
   // ---- deferred shading: once per (pixel, distinct winning triangle) -------
   uint32_t tid[N];
   if (VIS) {
-    // Samples that no triangle reached keep the surface's id.
+    // Samples that no triangle reached keep the surface's colour and id
+    // (first read here: deferred shading writes no colour before).
 #pragma unroll
     for (int i = 0; i < N; i++) {
+      col[i] = P.clearColor;
       tid[i] = 0xFFFFFFFFu;
-      if (!P.deferredClear && idOn && aux[i] == 0xFFFFFFFFu) tid[i] = triid[texelE + i * 8];
+    }
+    if (!P.deferredClear) {
+#pragma unroll
+      for (int i = 0; i < N; i++) {
+        col[i] = color[tileRowE + (laneE & 7) + i * 8];
+        if (idOn && aux[i] == 0xFFFFFFFFu) tid[i] = triid[tileRowE + (laneE & 7) + i * 8];
+      }
     }
     // Each pass shades the winner of this lane's first unresolved sample and
     // resolves every sample it won (aux -> ~0); a lane leaves when none is
@@ -692,9 +741,10 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
   const bool storeColor = blend != kBlendDepthOnly || P.deferredClear;
 #pragma unroll
   for (int i = 0; i < N; i++) {
-    if (storeColor) color[texelE + i * 8] = col[i];
-    depth[texelE + i * 8] = dep[i];
-    if (idOn) triid[texelE + i * 8] = tid[i];
+    const size_t at = tileRowE + (laneE & 7) + i * 8;
+    if (storeColor) color[at] = col[i];
+    depth[at] = dep[i];
+    if (idOn) triid[at] = tid[i];
   }
   // Fragment statistics only on counting draws: one plain store per tile
   // (a device-wide atomic per tile serialises across the XCDs).
@@ -765,9 +815,15 @@ __global__ void __launch_bounds__(64 * W, (fineMinWaves<S, VIS>()))
   const int g = banded ? xcdGroup(totalGroups) : (int)blockIdx.x;
   if (g >= totalGroups) return;
   const int k = findView(groupStart, numViews, g);
-  const Params& P = views[order[k]];
+  const Params* P = &views[order[k]];
   const int first = (g - groupStart[k]) * kFineRounds;
-  for (int t = 0; t < kFineRounds; t++) fineDispatch<S, VIS, false, W, DEPTH>(P, first + t, recAll);
+  for (int t = 0; t < kFineRounds; t++) {
+    // (Opaque: the parameters are not kept in registers from one round to
+    // the next.)
+    __asm__ volatile("" : "+s"(P));
+    const Params Q = loadParams(P);
+    fineDispatch<S, VIS, false, W, DEPTH>(Q, first + t, recAll);
+  }
 }
 
 // Variant v = (samplesLog2 * 2 + deferred shading) * 2 + depth test.

@@ -99,6 +99,10 @@ cr_status fail(cr_context* ctx, cr_status st, const char* fmt, ...);
 // (CudaRaster.cpp:174-179, base/Math.cpp:41-48, cuda/Util.hpp:290-298).
 void clearValues(const float rgba[4], float depth, uint32_t* color, uint32_t* encodedDepth);
 
+// Seconds per tick of the device's wall clock (asked for when times are: the
+// query takes tens of microseconds).
+double clockTick(int device);
+
 // setPixelPipe's checks of a pipe descriptor (CudaRaster.cpp:183-216).
 cr_status validatePipe(cr_context* ctx, const cr_pipe_desc* p);
 
@@ -185,7 +189,6 @@ struct cr_context {
   cr_profile_counters lastProf{};
   bool lastProfiled = false;                 // the last launch recorded profile counters
   bool drawn = false;                 // hostCounters hold (or will hold) a draw's stamps
-  double clockSeconds = 1e-8;         // one tick of the device's wall clock
   hipStream_t pendingStream = nullptr;
   hipEvent_t evPending = nullptr;     // after an asynchronous draw's counter readback
   bool pending = false;

@@ -623,7 +623,8 @@ __global__ void __launch_bounds__(kSetupChunk, 8) setupBinBatchKernel(const Para
                                                                    const int32_t* __restrict__ order,
                                                                    int numViews) {
   const int k = findView(blockStart, numViews, (int)blockIdx.x);
-  setupBinBody(views[order[k]], (int)blockIdx.x - blockStart[k]);
+  const Params P = loadParams(&views[order[k]]);
+  setupBinBody(P, (int)blockIdx.x - blockStart[k]);
 }
 
 void launchSetup(const Params& P, hipStream_t stream) {
