@@ -9,8 +9,8 @@
 // subtriangles take consecutive slots from a device counter (slots beyond
 // numTris), their source index goes to subtriTri, and misc holds the base.
 //
-// The clip polygon lives in registers (at most 9 vertices) instead of the
-// reference's per-thread shared-memory array.
+// The clip polygon lives in registers, one vertex per lane of the wave,
+// instead of the reference's per-thread shared-memory array.
 #include "cr_device.h"
 
 namespace crhip {
@@ -65,7 +65,9 @@ __device__ __forceinline__ uint32_t selectFlips(int32_t dx, int32_t dy) {
 // to the kernel's Params would make every wave copy the whole argument
 // block to scratch memory.
 struct ClipCtx {
-  int32_t viewportWidth, viewportHeight, samplesLog2, flags, shader, numTris, maxSubtris;
+  int32_t viewportWidth, viewportHeight, samplesLog2, flags, shader, numTris, maxSubtris, vertexStride;
+  const uint8_t* vertices;
+  const int32_t* indices;
   uint8_t* triSubtris;
   Header* triHeader;
   TriData* triData;
@@ -194,108 +196,148 @@ __device__ __forceinline__ void setupTriangle(const PP& P, Header* th, TriData* 
       (zmin & 0xFFFFF000u) | (f01 << 6) | (f12 << 2) | (f20 >> 2));
 }
 
-// clipPolygonWithPlane (Util.hpp:221-250), polygon in registers.
-__device__ __forceinline__ int clipPolygon(float* out, const float* in, int numIn, float v0, float v1, float v2) {
-  int numOut = 0;
-  if (numIn >= 3) {
-    int ai = (numIn - 1) * 2;
-    float av = fmaf(v2, in[ai + 1], fmaf(v1, in[ai + 0], v0));
-    for (int bi = 0; bi < numIn * 2; bi += 2) {
-      float bv = fmaf(v2, in[bi + 1], fmaf(v1, in[bi + 0], v0));
-      if (av * bv < 0.0f) {
-        float bc = av / (av - bv);
-        float ac = 1.0f - bc;
-        out[numOut + 0] = fmaf(in[ai + 0], ac, in[bi + 0] * bc);
-        out[numOut + 1] = fmaf(in[ai + 1], ac, in[bi + 1] * bc);
-        numOut += 2;
-      }
-      if (bv >= 0.0f) {
-        out[numOut + 0] = in[bi + 0];
-        out[numOut + 1] = in[bi + 1];
-        numOut += 2;
-      }
-      ai = bi;
-      av = bv;
-    }
+// ---- clipping: one triangle by the whole wave ---------------------------------
+//
+// Lane i holds vertex i of the clip polygon (at most 9) as its barycentrics;
+// vertices past the polygon's end take no part.  Few triangles are clipped,
+// so a wave clips them one after another: with a polygon per lane, in arrays
+// indexed at run time, a single clipped triangle held its 1024-triangle
+// workgroup up for 400k cycles of dependent scratch accesses (4M small
+// triangles among 1024 clipped ones, setup 382 -> 237 us with this and the
+// wide boxes below).
+struct ClipVert { float b0, b1; };
+
+// Vertex of lane `from`.
+__device__ __forceinline__ ClipVert vertOf(const ClipVert& v, int from) {
+  return {__shfl(v.b0, from, 64), __shfl(v.b1, from, 64)};
+}
+
+// clipPolygonWithPlane (Util.hpp:221-250): the polygon's part where
+// v0 + v1 b0 + v2 b1 >= 0.  Per vertex, in order: the intersection on the edge
+// that ends there, if any, then the vertex itself, if inside.
+__device__ __forceinline__ void clipPolygon(ClipVert& v, int& num, float v0, float v1, float v2) {
+  if (num < 3) {
+    num = 0;
+    return;
   }
-  return numOut >> 1;
+  const int lane = (int)(threadIdx.x & 63);
+  const ClipVert a = vertOf(v, lane == 0 ? num - 1 : lane - 1);
+  const float av = fmaf(v2, a.b1, fmaf(v1, a.b0, v0));
+  const float bv = fmaf(v2, v.b1, fmaf(v1, v.b0, v0));
+  const bool in = lane < num;
+  const bool cross = in && av * bv < 0.0f, keep = in && bv >= 0.0f;
+  const float bc = av / (av - bv);
+  const float ac = 1.0f - bc;
+  const ClipVert x = {fmaf(a.b0, ac, v.b0 * bc), fmaf(a.b1, ac, v.b1 * bc)};
+  const uint64_t cm = __ballot(cross), km = __ballot(keep);
+  // Output j: the (j + 1)-th of the marks, two per lane (cross, then keep).
+  // Each lane looks up the lane that its output comes from.
+  num = (int)(__popcll(cm) + __popcll(km));
+  int from = 0;
+  bool fromCross = false;
+  for (int q = 0, n = 0; q < 9; q++) {               // (at most 9 vertices: q is uniform)
+    const int c = (int)((cm >> q) & 1u), k = (int)((km >> q) & 1u);
+    if (c && n == lane) { from = q; fromCross = true; }
+    n += c;
+    if (k && n == lane) { from = q; fromCross = false; }
+    n += k;
+  }
+  const ClipVert fx = vertOf(x, from), fv = vertOf(v, from);
+  v = fromCross ? fx : fv;
 }
 
 __device__ __forceinline__ float comp(const float4& v, int a) { return a == 0 ? v.x : (a == 1 ? v.y : v.z); }
 
-// clipTriangleWithFrustum (Util.hpp:260-286)
-__device__ int clipTriangle(float bary[18], const float4& v0, const float4& v1, const float4& v2,
-                            const float4& d1, const float4& d2) {
+// clipTriangleWithFrustum (Util.hpp:260-286): returns the vertex count.
+__device__ __forceinline__ int clipTriangle(ClipVert& v, const float4& v0, const float4& v1, const float4& v2,
+                                            const float4& d1, const float4& d2) {
+  const int lane = (int)(threadIdx.x & 63);
   int num = 3;
-  bary[0] = 0.0f; bary[1] = 0.0f;
-  bary[2] = 1.0f; bary[3] = 0.0f;
-  bary[4] = 0.0f; bary[5] = 1.0f;
+  v = {lane == 1 ? 1.0f : 0.0f, lane == 2 ? 1.0f : 0.0f};
+#pragma unroll
   for (int a = 0; a < 3; a++) {
     if ((v0.w < fabsf(comp(v0, a))) | (v1.w < fabsf(comp(v1, a))) | (v2.w < fabsf(comp(v2, a)))) {
-      float temp[18];
-      num = clipPolygon(temp, bary, num, v0.w + comp(v0, a), d1.w + comp(d1, a), d2.w + comp(d2, a));
-      num = clipPolygon(bary, temp, num, v0.w - comp(v0, a), d1.w - comp(d1, a), d2.w - comp(d2, a));
+      clipPolygon(v, num, v0.w + comp(v0, a), d1.w + comp(d1, a), d2.w + comp(d2, a));
+      clipPolygon(v, num, v0.w - comp(v0, a), d1.w - comp(d1, a), d2.w - comp(d2, a));
     }
   }
   return num;
 }
 
-__device__ __forceinline__ float4 lerpClip(const float4& o, const float4& d1, const float4& d2, float b0, float b1) {
-  return make_float4(fmaf(d2.x, b1, fmaf(d1.x, b0, o.x)), fmaf(d2.y, b1, fmaf(d1.y, b0, o.y)),
-                     fmaf(d2.z, b1, fmaf(d1.z, b0, o.z)), fmaf(d2.w, b1, fmaf(d1.w, b0, o.w)));
+__device__ __forceinline__ float4 lerpClip(const float4& o, const float4& d1, const float4& d2, const ClipVert& b) {
+  return make_float4(fmaf(d2.x, b.b1, fmaf(d1.x, b.b0, o.x)), fmaf(d2.y, b.b1, fmaf(d1.y, b.b0, o.y)),
+                     fmaf(d2.z, b.b1, fmaf(d1.z, b.b0, o.z)), fmaf(d2.w, b.b1, fmaf(d1.w, b.b0, o.w)));
 }
 
-// Slow path, kept out of line: frustum clip and fan (TriangleSetup.inl:326-412).
-// Returns the number of subtriangles written (0 when the slot allocation
-// overflowed) and their first slot in *baseOut.
-__device__ __noinline__ int setupClipped(const ClipCtx P, int t, int3 vidx, float4 v0, float4 v1, float4 v2,
-                                         int* baseOut) {
-  float4 od1 = make_float4(v1.x - v0.x, v1.y - v0.y, v1.z - v0.z, v1.w - v0.w);
-  float4 od2 = make_float4(v2.x - v0.x, v2.y - v0.y, v2.z - v0.z, v2.w - v0.w);
-  float4 ov0 = v0;
-  float bary[18];
-  int numVerts = clipTriangle(bary, ov0, v1, v2, od1, od2);
-  v0 = lerpClip(ov0, od1, od2, bary[0], bary[1]);
-  v1 = lerpClip(ov0, od1, od2, bary[2], bary[3]);
-  float4 tv1 = v1;
-  I2 p0, p1, p2, lo, hi, d1, d2;
-  float rcpW[3];
-  int32_t area;
+__device__ __forceinline__ float4 laneValue(const float4& v, int j) {
+  return make_float4(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v.x), j)),
+                     __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v.y), j)),
+                     __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v.z), j)),
+                     __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v.w), j)));
+}
 
-  int numSub = 0;
-  for (int i = 2; i < numVerts; i++) {
-    float4 vv2 = lerpClip(ov0, od1, od2, bary[i * 2], bary[i * 2 + 1]);
-    snap(P, v0, v1, vv2, p0, p1, p2, rcpW, lo, hi);
-    if (prepare(P, p0, p1, p2, lo, hi, d1, d2, area) == 0) numSub++;
-    v1 = vv2;
+struct ClipResult { int numSub, base; };
+
+// Slow path, kept out of line, called by whole waves: frustum clip and fan
+// (TriangleSetup.inl:326-412) of the triangles of the lanes in `todo`, one
+// after another; lane f sets up fan triangle f.  Returns, per lane in todo,
+// the number of subtriangles written (0 when the slot allocation overflowed)
+// and their first slot.
+__device__ __noinline__ ClipResult setupClipped(const ClipCtx P, uint64_t todo, int tOwn) {
+  const int lane = (int)(threadIdx.x & 63);
+  ClipResult out = {0, tOwn};
+  int3 vidxOwn = make_int3(0, 0, 0);
+  float4 own0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), own1 = own0, own2 = own0;
+  if ((todo >> lane) & 1u) {
+    const int32_t* ip = P.indices + (int64_t)tOwn * 3;
+    vidxOwn = make_int3(ip[0], ip[1], ip[2]);
+    own0 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidxOwn.x * P.vertexStride);
+    own1 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidxOwn.y * P.vertexStride);
+    own2 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidxOwn.z * P.vertexStride);
   }
-  P.triSubtris[t] = (uint8_t)numSub;
-
-  int base = t;
-  if (numSub > 1) {
-    base = P.numTris + (int)atomicAdd(&P.counters->numSubtris, (uint32_t)numSub);
-    P.triHeader[t].misc = (uint32_t)base;
-    if (base + numSub > P.maxSubtris) {
-      atomicOr(&P.counters->overflow, 1u);
-      numVerts = 0;
-      numSub = 0;
+  for (; todo != 0; todo &= todo - 1) {
+    const int j = (int)__builtin_ctzll(todo);
+    const int t = __builtin_amdgcn_readlane(tOwn, j);
+    const int3 vidx = make_int3(__builtin_amdgcn_readlane(vidxOwn.x, j), __builtin_amdgcn_readlane(vidxOwn.y, j),
+                                __builtin_amdgcn_readlane(vidxOwn.z, j));
+    const float4 ov0 = laneValue(own0, j), ov1 = laneValue(own1, j), ov2 = laneValue(own2, j);
+    const float4 od1 = make_float4(ov1.x - ov0.x, ov1.y - ov0.y, ov1.z - ov0.z, ov1.w - ov0.w);
+    const float4 od2 = make_float4(ov2.x - ov0.x, ov2.y - ov0.y, ov2.z - ov0.z, ov2.w - ov0.w);
+    ClipVert v;
+    const int numVerts = clipTriangle(v, ov0, ov1, ov2, od1, od2);
+    const ClipVert c0 = vertOf(v, 0), c1 = vertOf(v, (lane + 1) & 63), c2 = vertOf(v, (lane + 2) & 63);
+    const float4 v0 = lerpClip(ov0, od1, od2, c0), v1 = lerpClip(ov0, od1, od2, c1), v2 = lerpClip(ov0, od1, od2, c2);
+    I2 p0, p1, p2, lo, hi, d1, d2;
+    float rcpW[3];
+    int32_t area;
+    snap(P, v0, v1, v2, p0, p1, p2, rcpW, lo, hi);
+    const bool vis = lane + 2 < numVerts && prepare(P, p0, p1, p2, lo, hi, d1, d2, area) == 0;
+    const uint64_t vm = __ballot(vis);
+    int numSub = (int)__popcll(vm);
+    int base = t;
+    if (numSub > 1) {
+      int at = 0;
+      if (lane == 0) at = P.numTris + (int)atomicAdd(&P.counters->numSubtris, (uint32_t)numSub);
+      base = __builtin_amdgcn_readfirstlane(at);
+    }
+    const bool over = numSub > 1 && base + numSub > P.maxSubtris;
+    if (lane == 0) {
+      P.triSubtris[t] = (uint8_t)numSub;
+      if (numSub > 1) P.triHeader[t].misc = (uint32_t)base;
+      if (over) atomicOr(&P.counters->overflow, 1u);
+    }
+    if (vis && !over) {
+      const int slot = base + (int)__popcll(vm & ((1ull << lane) - 1ull));
+      setupTriangle(P, &P.triHeader[slot], &P.triData[slot], vidx, v0, v1, v2, make_float2(c0.b0, c0.b1),
+                    make_float2(c1.b0, c1.b1), make_float2(c2.b0, c2.b1), p0, p1, p2, rcpW, d1, d2, area);
+      if (slot >= P.numTris) P.subtriTri[slot - P.numTris] = (uint32_t)t;
+    }
+    if (lane == j) {
+      out.numSub = over ? 0 : numSub;
+      out.base = base;
     }
   }
-  *baseOut = base;
-  v1 = tv1;
-  for (int i = 2; i < numVerts; i++) {
-    float4 vv2 = lerpClip(ov0, od1, od2, bary[i * 2], bary[i * 2 + 1]);
-    snap(P, v0, v1, vv2, p0, p1, p2, rcpW, lo, hi);
-    if (prepare(P, p0, p1, p2, lo, hi, d1, d2, area) == 0) {
-      setupTriangle(P, &P.triHeader[base], &P.triData[base], vidx, v0, v1, vv2,
-                    make_float2(bary[0], bary[1]), make_float2(bary[i * 2 - 2], bary[i * 2 - 1]),
-                    make_float2(bary[i * 2], bary[i * 2 + 1]), p0, p1, p2, rcpW, d1, d2, area);
-      if (base >= P.numTris) P.subtriTri[base - P.numTris] = (uint32_t)t;
-      base++;
-    }
-    v1 = vv2;
-  }
-  return numSub;
+  return out;
 }
 
 // Outcome of one triangle's setup, as the reference's setup counters
@@ -303,12 +345,13 @@ __device__ __noinline__ int setupClipped(const ClipCtx P, int t, int3 vidx, floa
 enum SetupOutcome : int { kSetupVisible = 0, kSetupFrustum, kSetupBackface, kSetupBetween, kSetupClipPath,
                           kSetupDropped };
 
-// One triangle: returns its number of subtriangles and their first slot.
-// When the triangle is set up without clipping, *hv receives the header's
-// vertex words (as written to P.triHeader[t]) and *hvOk is set.  *why
-// receives the SetupOutcome.
-__device__ __forceinline__ int setupOne(const Params& P, int t, int* base, uint4* hv, bool* hvOk, int* why) {
-  *base = t;
+// One triangle: returns its number of subtriangles (in slot t).  When the
+// triangle is set up without clipping, *hv receives the header's vertex words
+// (as written to P.triHeader[t]) and *hvOk is set.  *why receives the
+// SetupOutcome; kSetupClipPath leaves the triangle to setupClipped, its
+// vertices to be read again there (kept in registers, they would cost every
+// wave).
+__device__ __forceinline__ int setupOne(const Params& P, int t, uint4* hv, bool* hvOk, int* why) {
   *hvOk = false;
   *why = kSetupDropped;
   int3 vidx;
@@ -321,9 +364,9 @@ __device__ __forceinline__ int setupOne(const Params& P, int t, int* base, uint4
     P.triSubtris[t] = 0;
     return 0;
   }
-  float4 v0 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.x * P.vertexStride);
-  float4 v1 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.y * P.vertexStride);
-  float4 v2 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.z * P.vertexStride);
+  const float4 v0 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.x * P.vertexStride);
+  const float4 v1 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.y * P.vertexStride);
+  const float4 v2 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.z * P.vertexStride);
 
   // Outside view frustum => cull (:262-281).
   if ((v0.w < fabsf(v0.x)) | (v0.w < fabsf(v0.y)) | (v0.w < fabsf(v0.z))) {
@@ -365,9 +408,7 @@ __device__ __forceinline__ int setupOne(const Params& P, int t, int* base, uint4
     }
   }
   *why = kSetupClipPath;
-  const ClipCtx C = {P.viewportWidth, P.viewportHeight, P.samplesLog2, (int32_t)P.flags, P.shader,
-                     P.numTris, P.maxSubtris, P.triSubtris, P.triHeader, P.triData, P.subtriTri, P.counters};
-  return setupClipped(C, t, vidx, v0, v1, v2, base);
+  return 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -408,62 +449,85 @@ __device__ __forceinline__ BinBox binBoxOf(const Params& P, uint4 h) {
   return b;
 }
 
+// Boxes of more bins than this are walked by their whole wave, 16 x 4 bins at
+// a time, instead of by their own lane bin by bin (a full-screen triangle's
+// 256 bins held its workgroup up for 150k cycles).
+constexpr int kCoopBins = 6;
+
+// Calls f(bin, j) for every bin of lane j's box (j uniform).
+template <class F>
+__device__ __forceinline__ void forEachBinCoop(const Params& P, const BinBox& b, int j, F&& f) {
+  const int lane = (int)(threadIdx.x & 63);
+  const int x0 = __builtin_amdgcn_readlane(b.x0, j), x1 = __builtin_amdgcn_readlane(b.x1, j);
+  const int y0 = __builtin_amdgcn_readlane(b.y0, j), y1 = __builtin_amdgcn_readlane(b.y1, j);
+  for (int ys = y0; ys <= y1; ys += 4)
+    for (int xs = x0; xs <= x1; xs += 16) {
+      const int x = xs + (lane & 15), y = ys + (lane >> 4);
+      if (x <= x1 && y <= y1) f(x + y * P.widthBins, j);
+    }
+}
+
 __device__ __forceinline__ uint64_t laneLt() {
   const uint32_t lane = threadIdx.x & 63;
   return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
-// Exclusive scan of one value per thread over the whole block.
+// Exclusive scan of one value per thread over the whole block (at most 16
+// waves: every wave adds up the wave sums by itself).  One barrier; a scan
+// that may follow without another needs `sums` of its own.
 template <int NT>
 __device__ __forceinline__ uint32_t blockScan(uint32_t v, uint32_t* sums, uint32_t& total) {
   constexpr int NW = NT / 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
+  static_assert(NW <= 16, "one row of lanes holds the wave sums");
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t x = waveScan(v);
   if (lane == 63) sums[wave] = x;
   __syncthreads();
-  if (threadIdx.x < 64) {
-    const uint32_t w = (threadIdx.x < NW) ? sums[threadIdx.x] : 0u;
-    uint32_t sc = w;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t y = __shfl_up(sc, o, 64);
-      if ((int)threadIdx.x >= o) sc += y;
-    }
-    if (threadIdx.x < NW) sums[threadIdx.x] = sc - w;
-    if (threadIdx.x == NW - 1) sums[NW] = sc;
-  }
-  __syncthreads();
-  total = sums[NW];
-  const uint32_t r = sums[wave] + x - v;
-  __syncthreads();
-  return r;
+  const uint32_t w = lane < NW ? sums[lane] : 0u;
+  const uint32_t sc = waveScan(w);
+  total = (uint32_t)__builtin_amdgcn_readlane((int)sc, NW - 1);
+  const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(sc - w), wave);
+  return before + x - v;
 }
 
 // Setup and binning of chunk `chunk` of one draw (one 1024-lane workgroup).
-__device__ __forceinline__ void setupBinBody(const Params& P, const int chunk) {
+// load(): the draw's parameters; asked for once by the setup and once by the
+// binning, so that a batch, which loads them from its table, need not hold
+// the one's through the other.
+template <class Load>
+__device__ __forceinline__ void setupBinBody(Load&& load, const int chunk) {
   __shared__ uint32_t cnt[kMaxBins];
   __shared__ uint32_t run[kMaxBins];
   __shared__ uint64_t emitMask[kSetupWaves][kMaxBins];
   __shared__ uint32_t emitPre[kSetupWaves][kMaxBins];
   __shared__ uint32_t list[kSetupChunk];
-  __shared__ uint32_t sums[kSetupWaves + 1];
+  __shared__ uint32_t sums[2][kSetupWaves];
   __shared__ uint32_t sBase;
   __shared__ uint32_t sProf[8];
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int t = chunk * kSetupChunk + threadIdx.x;
-  if (chunk == 0) stampStage(P, kStampSetup);
-
   // ---- setup ---------------------------------------------------------------
   int base = t, k = 0, why = kSetupDropped;
   uint4 hvOwn = make_uint4(0u, 0u, 0u, 0u);   // header vertex words kept from setup (no re-read)
   bool hvOwnOk = false;
-  if (t < P.numTris) k = setupOne(P, t, &base, &hvOwn, &hvOwnOk, &why);
+  {
+    auto&& P = load();
+    if (chunk == 0) stampStage(P, kStampSetup);
+    if (t < P.numTris) k = setupOne(P, t, &hvOwn, &hvOwnOk, &why);
+    const uint64_t clip = __ballot(t < P.numTris && why == kSetupClipPath);
+    if (__builtin_expect(clip != 0, 0)) {
+      const ClipCtx C = {P.viewportWidth, P.viewportHeight, P.samplesLog2, (int32_t)P.flags, P.shader,
+                         P.numTris, P.maxSubtris, P.vertexStride, P.vertices, P.indices, P.triSubtris, P.triHeader,
+                         P.triData, P.subtriTri, P.counters};
+      const ClipResult r = setupClipped(C, clip, t);
+      if ((clip >> lane) & 1u) {
+        k = r.numSub;
+        base = r.base;
+      }
+    }
+  }
+  auto&& P = load();
   if (P.prof != nullptr) {
     // Profiling draws: per-outcome triangle counts of the chunk, then its
     // triangles with at least one subtriangle.
@@ -499,7 +563,7 @@ __device__ __forceinline__ void setupBinBody(const Params& P, const int chunk) {
   // submission order; a chunk without clipped triangles is a single window.
   const bool compact = __syncthreads_or(k > 1) != 0;
   uint32_t total;
-  const uint32_t pos = blockScan<kSetupChunk>((uint32_t)k, sums, total);
+  const uint32_t pos = blockScan<kSetupChunk>((uint32_t)k, sums[0], total);
   const uint32_t numWin = (total + kSetupChunk - 1) / kSetupChunk;
   if (P.chunkSubtris != nullptr && threadIdx.x == 0) P.chunkSubtris[chunk] = total;
 
@@ -533,9 +597,16 @@ __device__ __forceinline__ void setupBinBody(const Params& P, const int chunk) {
       }
     }
     const uint64_t bit = 1ull << lane;
-    for (int y = bb.y0; y <= bb.y1; y++)
-      for (int x = bb.x0; x <= bb.x1; x++)
-        atomicOr((unsigned long long*)&emitMask[wave][x + y * P.widthBins], (unsigned long long)bit);
+    const bool big = (bb.x1 - bb.x0 + 1) * (bb.y1 - bb.y0 + 1) > kCoopBins && bb.x0 <= bb.x1;
+    if (!big) {
+      for (int y = bb.y0; y <= bb.y1; y++)
+        for (int x = bb.x0; x <= bb.x1; x++)
+          atomicOr((unsigned long long*)&emitMask[wave][x + y * P.widthBins], (unsigned long long)bit);
+    }
+    for (uint64_t m = __ballot(big); m != 0; m &= m - 1)
+      forEachBinCoop(P, bb, (int)__builtin_ctzll(m), [&](int bin, int j) {
+        atomicOr((unsigned long long*)&emitMask[wave][bin], 1ull << j);
+      });
     __syncthreads();
     return true;
   };
@@ -563,7 +634,7 @@ __device__ __forceinline__ void setupBinBody(const Params& P, const int chunk) {
   // ---- reserve the chunk's region; publish counts and offsets ---------------
   uint32_t tot2;
   const uint32_t c = (threadIdx.x < (unsigned)P.numBins) ? cnt[threadIdx.x] : 0u;
-  const uint32_t off = blockScan<kSetupChunk>(c, sums, tot2);
+  const uint32_t off = blockScan<kSetupChunk>(c, sums[1], tot2);
   if (P.prof != nullptr && threadIdx.x == 0) {
     profAdd(P.prof, kProfBinTrisPerChunk, total, 1);
     profAdd(P.prof, kProfBinTriBBArea, tot2, total);
@@ -603,18 +674,30 @@ __device__ __forceinline__ void setupBinBody(const Params& P, const int chunk) {
       run[i] = acc;
     }
     __syncthreads();
-    const uint64_t lt = laneLt();
-    for (int y = bb.y0; y <= bb.y1; y++)
-      for (int x = bb.x0; x <= bb.x1; x++) {
-        const int bin = x + y * P.widthBins;
-        const uint32_t p = regionBase + emitPre[wave][bin] + (uint32_t)__popcll(emitMask[wave][bin] & lt);
-        if (p < (uint32_t)P.maxBinEntries) P.binList[p] = make_uint4(slot, hv.x, hv.y, hv.z);
-      }
+    auto put = [&](int bin, uint64_t lt, const uint4& e) {
+      const uint32_t p = regionBase + emitPre[wave][bin] + (uint32_t)__popcll(emitMask[wave][bin] & lt);
+      if (p < (uint32_t)P.maxBinEntries) P.binList[p] = e;
+    };
+    const uint4 e = make_uint4(slot, hv.x, hv.y, hv.z);
+    const bool big = (bb.x1 - bb.x0 + 1) * (bb.y1 - bb.y0 + 1) > kCoopBins && bb.x0 <= bb.x1;
+    if (!big) {
+      const uint64_t lt = laneLt();
+      for (int y = bb.y0; y <= bb.y1; y++)
+        for (int x = bb.x0; x <= bb.x1; x++) put(x + y * P.widthBins, lt, e);
+    }
+    for (uint64_t m = __ballot(big); m != 0; m &= m - 1) {
+      const int j = (int)__builtin_ctzll(m);
+      const uint4 ej = make_uint4(__builtin_amdgcn_readlane(e.x, j), __builtin_amdgcn_readlane(e.y, j),
+                                  __builtin_amdgcn_readlane(e.z, j), __builtin_amdgcn_readlane(e.w, j));
+      forEachBinCoop(P, bb, j, [&](int bin, int l) { put(bin, (1ull << l) - 1ull, ej); });
+    }
     __syncthreads();
   }
 }
 
-__global__ void __launch_bounds__(kSetupChunk, 8) setupBinKernel(const Params P) { setupBinBody(P, blockIdx.x); }
+__global__ void __launch_bounds__(kSetupChunk, 8) setupBinKernel(const Params P) {
+  setupBinBody([&]() -> const Params& { return P; }, blockIdx.x);
+}
 
 // Batched draws: one workgroup per chunk of every view; blockStart[v] is the
 // first workgroup of view v (numViews + 1 entries).
@@ -623,8 +706,13 @@ __global__ void __launch_bounds__(kSetupChunk, 8) setupBinBatchKernel(const Para
                                                                    const int32_t* __restrict__ order,
                                                                    int numViews) {
   const int k = findView(blockStart, numViews, (int)blockIdx.x);
-  const Params P = loadParams(&views[order[k]]);
-  setupBinBody(P, (int)blockIdx.x - blockStart[k]);
+  const Params* view = &views[order[k]];
+  setupBinBody(
+      [&]() {
+        __asm__ volatile("" : "+s"(view));
+        return loadParams(view);
+      },
+      (int)blockIdx.x - blockStart[k]);
 }
 
 void launchSetup(const Params& P, hipStream_t stream) {
