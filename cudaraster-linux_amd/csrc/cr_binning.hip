@@ -41,36 +41,6 @@ __device__ __forceinline__ uint32_t rankBelow(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-template <int NT>
-__device__ __forceinline__ uint32_t blockScanC(uint32_t v, uint32_t* sums, uint32_t& total) {
-  constexpr int NW = NT / 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) sums[wave] = x;
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    const uint32_t w = (threadIdx.x < NW) ? sums[threadIdx.x] : 0u;
-    uint32_t sc = w;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t y = __shfl_up(sc, o, 64);
-      if ((int)threadIdx.x >= o) sc += y;
-    }
-    if (threadIdx.x < NW) sums[threadIdx.x] = sc - w;
-    if (threadIdx.x == NW - 1) sums[NW] = sc;
-  }
-  __syncthreads();
-  total = sums[NW];
-  const uint32_t r = sums[wave] + x - v;
-  __syncthreads();
-  return r;
-}
-
 // Clears the counter block (and a profiling draw's profile counters) with
 // plain stores: graph-safe, no memset node.  Only for draws that cannot rely
 // on the draw before them having left the block cleared.
@@ -122,6 +92,27 @@ struct TileTest {
   }
 };
 
+// The same test tile after tile of a walk in rows: what each edge's left side
+// exceeds its threshold by, stepped by additions (a 32-bit product takes four
+// times as long as an addition).  Within 15 tiles of the box each value stays
+// below 2^30 + 2^30.
+struct TileWalk {
+  int32_t e[3], row[3];
+  __device__ __forceinline__ TileWalk(const TileTest& r, int x, int y) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) e[k] = row[k] = (x - r.x0) * r.sx[k] + (y - r.y0) * r.sy[k] - r.G[k];
+  }
+  __device__ __forceinline__ bool hit() const { return max(max(e[0], e[1]), e[2]) <= 0; }
+  __device__ __forceinline__ void right(const TileTest& r) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) e[k] += r.sx[k];
+  }
+  __device__ __forceinline__ void nextRow(const TileTest& r) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) e[k] = row[k] = row[k] + r.sy[k];
+  }
+};
+
 // Tile (x, y) of the bin holds a covered sample only if its closed square
 // reaches the inner side of all three edges: min over the square of
 // p x d <= a x d.  With the corner that minimises p x d, p x d at tile
@@ -144,15 +135,14 @@ __device__ __forceinline__ TileTest tileTestOf(const Params& P, uint4 h, int bx,
   const int32_t lastY = min(P.heightTiles - ty0, 1 << bl) - 1;
   r.x0 = max((minx >> ts) - tx0, 0); r.x1 = min((maxx >> ts) - tx0, lastX);
   r.y0 = max((miny >> ts) - ty0, 0); r.y1 = min((maxy >> ts) - ty0, lastY);
-  const int64_t BX = (int64_t)(tx0 + r.x0) << ts, BY = (int64_t)(ty0 + r.y0) << ts;
+  const int32_t BX = (tx0 + r.x0) << ts, BY = (ty0 + r.y0) << ts;
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     const int j = (k + 1) % 3;
     const int32_t dx = ax[j] - ax[k], dy = ay[j] - ay[k];
-    const int64_t c = (int64_t)ax[k] * dy - (int64_t)ay[k] * dx;
-    const int64_t px = BX + ((dy > 0) ? 0 : (1 << ts));
-    const int64_t py = BY + ((dx > 0) ? (1 << ts) : 0);
-    int64_t g = c - (px * dy - py * dx);
+    const int32_t px = BX + ((dy > 0) ? 0 : (1 << ts));
+    const int32_t py = BY + ((dx > 0) ? (1 << ts) : 0);
+    int64_t g = (int64_t)(ax[k] - px) * dy - (int64_t)(ay[k] - py) * dx;   // (a - p) x d
     g = g > (1ll << 30) ? (1ll << 30) : (g < -(1ll << 30) ? -(1ll << 30) : g);
     r.G[k] = (int32_t)g;
     r.sx[k] = dy * (1 << ts);
@@ -231,14 +221,17 @@ __device__ __forceinline__ TileTest getBig(const BigEntry* e, uint32_t& slot, ui
 // whichever waves are free, spreading them over the workgroup.  A large box
 // that reaches every tile of a complete bin (*whole) sets no mask bits: its
 // wave's word fullBits[wave] holds it for every tile, and its slot goes to
-// wholeSlot[wave * 64 + lane] for the writes.  Returns the CoarseCase the
-// wave took.
+// wholeSlot[wave * 64 + lane] for the writes.  hits: the tiles of a small box
+// that the entry reaches, bit i the i-th of its box row by row.  Returns the
+// CoarseCase the wave took.
 __device__ __forceinline__ int coarseRecord(const TileTest& r, bool valid, const int bl,
                                             uint64_t (*emitMask)[kBinTiles], BigEntry* big,
                                             uint32_t* bigCount, uint32_t bigCap, uint32_t slot,
                                             bool& queued, bool binComplete, uint64_t* fullBits,
-                                            uint32_t* wholeSlot, uint32_t* wholeCount, bool& whole) {
+                                            uint32_t* wholeSlot, uint32_t* wholeCount, bool& whole,
+                                            uint32_t& hits) {
   queued = false;
+  hits = 0;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   int w = valid ? r.x1 - r.x0 + 1 : 0, h = valid ? r.y1 - r.y0 + 1 : 0;
   // Every tile of the bin hit: the box is the bin and the tile test's left
@@ -275,25 +268,25 @@ __device__ __forceinline__ int coarseRecord(const TileTest& r, bool valid, const
     // LDS atomic that lanes hitting the same tile serialise: weight 2), plus
     // one wave step per 64 tiles for each large box.
     const bool bigOne = has && w * h > kCoopArea;
-    int a0 = has ? r.x0 : 1 << 20, a1 = has ? r.x1 : -1, b0 = has ? r.y0 : 1 << 20, b1 = has ? r.y1 : -1;
-    int smallArea = (has && !bigOne) ? w * h : 0;
-    int bigSteps = bigOne ? (h + 3) >> 2 : 0;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      a0 = min(a0, __shfl_xor(a0, o, 64)); a1 = max(a1, __shfl_xor(a1, o, 64));
-      b0 = min(b0, __shfl_xor(b0, o, 64)); b1 = max(b1, __shfl_xor(b1, o, 64));
-      smallArea = max(smallArea, __shfl_xor(smallArea, o, 64));
-      bigSteps += __shfl_xor(bigSteps, o, 64);
-    }
-    ux0 = a0; ux1 = a1; uy0 = b0; uy1 = b1;
+    const int smallArea = waveReduce((has && !bigOne) ? w * h : 0, 0, [](int a, int b) { return max(a, b); });
+    const int bigSteps = waveReduce(bigOne ? (h + 3) >> 2 : 0, 0, [](int a, int b) { return a + b; });
+    ux0 = waveReduce(has ? r.x0 : 1 << 20, 1 << 20, [](int a, int b) { return min(a, b); });
+    ux1 = waveReduce(has ? r.x1 : -1, -1, [](int a, int b) { return max(a, b); });
+    uy0 = waveReduce(has ? r.y0 : 1 << 20, 1 << 20, [](int a, int b) { return min(a, b); });
+    uy1 = waveReduce(has ? r.y1 : -1, -1, [](int a, int b) { return max(a, b); });
     coop = (ux1 - ux0 + 1) * (uy1 - uy0 + 1) <= 2 * smallArea + bigSteps;
   }
   if (coop) {
-    for (int y = uy0; y <= uy1; y++)
-      for (int x = ux0; x <= ux1; x++) {
-        const bool hit = has && x >= r.x0 && x <= r.x1 && y >= r.y0 && y <= r.y1 && r.hit(x, y);
+    TileWalk tw(r, ux0, uy0);
+    uint32_t at = has && w * h <= kCoopArea ? 1u : 0u;     // the next tile of this lane's box
+    for (int y = uy0; y <= uy1; y++, tw.nextRow(r))
+      for (int x = ux0; x <= ux1; x++, tw.right(r)) {
+        const bool inBox = has && x >= r.x0 && x <= r.x1 && y >= r.y0 && y <= r.y1;
+        const bool hit = inBox && tw.hit();
         const uint64_t m = __ballot(hit);
         if (m != 0 && lane == 0) emitMask[wave][x + (y << bl)] = m;
+        hits |= hit ? at : 0u;
+        at <<= inBox ? 1 : 0;
       }
     return kCaseB;
   }
@@ -314,10 +307,21 @@ __device__ __forceinline__ int coarseRecord(const TileTest& r, bool valid, const
   if (has && !isBig) {
     // One loop over the box (row by row): as many wave steps as the
     // largest small box has tiles.
-    int x = r.x0, y = r.y0;
+    int x = r.x0, ti = r.x0 + (r.y0 << bl);
+    TileWalk tw(r, r.x0, r.y0);
     for (int i = 0; i < w * h; i++) {
-      if (r.hit(x, y)) atomicOr((unsigned long long*)&emitMask[wave][x + (y << bl)], (unsigned long long)bit);
-      if (++x > r.x1) { x = r.x0; y++; }
+      if (tw.hit()) {
+        atomicOr((unsigned long long*)&emitMask[wave][ti], (unsigned long long)bit);
+        hits |= 1u << i;
+      }
+      if (++x > r.x1) {
+        x = r.x0;
+        ti += (1 << bl) - (w - 1);
+        tw.nextRow(r);
+      } else {
+        ti++;
+        tw.right(r);
+      }
     }
   }
   for (uint64_t b = __ballot(isBig && !queued); b != 0; b &= b - 1) {
@@ -399,7 +403,7 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
     if (i0 < nb) segAddr[i0] = P.chunkBase[cb + i0] + bOff[cb + i0];
     if (i1 < nb) segAddr[i1] = P.chunkBase[cb + i1] + bOff[cb + i1];
     uint32_t segTotal;
-    const uint32_t s0 = blockScanC<kCoarseThreads>(n0 + n1, sums, segTotal);
+    const uint32_t s0 = blockScan<kCoarseThreads>(n0 + n1, sums, segTotal);
     if (i0 < nb) segStart[i0] = s0;
     if (i1 < nb) segStart[i1] = s0 + n0;
     if (threadIdx.x == 0) segStart[nb] = segTotal;
@@ -445,8 +449,9 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
         if (valid) r = tileTestOf(P, make_uint4(e.y, e.z, e.w, 0u), bx, by);
       }
       bool queued, whole;
+      uint32_t hits;
       const int wcase = coarseRecord(r, valid, bl, emitMask, bigQ, &sBigCount, kBigCap, slot, queued, binComplete,
-                                     sFull, wholeSlot, &sWholeCount, whole);
+                                     sFull, wholeSlot, &sWholeCount, whole, hits);
       if (g + kCoarseThreads < segTotal) eNext = entryAt(g + kCoarseThreads);
       if (prof) {
         const uint32_t nv = (uint32_t)__popcll(__ballot(valid));
@@ -508,12 +513,7 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
       // 256: the first four waves) scan their segment needs -- a wave scan,
       // then the four wave totals -- so the reservation costs two barriers.
       static_assert(kBinTiles <= 256 && kCoarseWaves >= 4, "tiles in the first four waves");
-      uint32_t x = need;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-      }
+      const uint32_t x = waveScan(need);
       if (wave < 4 && lane == 63) sums[wave] = x;
       __syncthreads();
       const uint32_t w0 = sums[0], w1 = sums[1], w2 = sums[2], w3 = sums[3];
@@ -571,21 +571,17 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
         if (sg < segCap) P.tileList[((size_t)sg << kTileSegLog2) + (e & (kTileSeg - 1))] = sl;
       };
       const bool hasBox = valid && !whole && r.x0 <= r.x1 && r.y0 <= r.y1;
-      const int boxArea = hasBox ? (r.x1 - r.x0 + 1) * (r.y1 - r.y0 + 1) : 0;
-      const bool bigBox = boxArea > kCoopArea;
-      if (hasBox && !bigBox) {
-        const uint64_t bit = 1ull << lane;
-        // One loop over the box (row by row): the wave runs as many steps
-        // as its largest box has tiles.
-        int x = r.x0, y = r.y0;
-        for (int i = 0; i < boxArea; i++) {
-          const int ti = x + (y << bl);
-          const uint64_t m = emitMask[wave][ti];
-          const uint32_t pre = emitPre[wave][ti];
-          const uint4 q = tRound[ti];
-          if (m & bit) put(q, pre + rankBelow(m), slot);
-          if (++x > r.x1) { x = r.x0; y++; }
-        }
+      const int boxW = r.x1 - r.x0 + 1;
+      const bool bigBox = hasBox && boxW * (r.y1 - r.y0 + 1) > kCoopArea;
+      // Small boxes: the tiles that the entry reaches, so that the wave runs
+      // as many steps as its widest-spread entry reaches tiles.  Tile i of a
+      // box is in row i / boxW: (i * ceil(256 / boxW)) >> 8 for i < 16.
+      const uint32_t inv = boxW > 1 ? (uint32_t)(256.0f * __builtin_amdgcn_rcpf((float)boxW) + 0.999f) : 256u;
+      for (uint32_t m = hits; m != 0; m &= m - 1) {
+        const uint32_t i = (uint32_t)__builtin_ctz(m);
+        const uint32_t row = (i * inv) >> 8;
+        const int ti = r.x0 + (int)(i - row * (uint32_t)boxW) + ((r.y0 + (int)row) << bl);
+        put(tRound[ti], emitPre[wave][ti] + rankBelow(emitMask[wave][ti]), slot);
       }
       for (uint64_t b = __ballot(bigBox && !queued); b != 0; b &= b - 1) {
         const int j = (int)__builtin_ctzll(b);

@@ -374,6 +374,36 @@ __device__ __forceinline__ uint32_t waveScan(uint32_t v) {
   return v;
 }
 
+// The operation over the wave's lanes, in every lane (DPP steps as above).
+template <class Op>
+__device__ __forceinline__ int32_t waveReduce(int32_t v, int32_t identity, Op op) {
+  v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x111, 0xF, 0xF, false));
+  v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x112, 0xF, 0xF, false));
+  v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x114, 0xF, 0xF, false));
+  v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x118, 0xF, 0xF, false));
+  v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x142, 0xA, 0xF, false));
+  v = op(v, __builtin_amdgcn_update_dpp(identity, v, 0x143, 0xC, 0xF, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// Exclusive scan of one value per thread over the whole block (at most 16
+// waves: every wave adds up the wave sums by itself).  One barrier; a scan
+// that may follow without another needs `sums` of its own.
+template <int NT>
+__device__ __forceinline__ uint32_t blockScan(uint32_t v, uint32_t* sums, uint32_t& total) {
+  constexpr int NW = NT / 64;
+  static_assert(NW <= 16, "one row of lanes holds the wave sums");
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t x = waveScan(v);
+  if (lane == 63) sums[wave] = x;
+  __syncthreads();
+  const uint32_t w = lane < NW ? sums[lane] : 0u;
+  const uint32_t sc = waveScan(w);
+  total = (uint32_t)__builtin_amdgcn_readlane((int)sc, NW - 1);
+  const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(sc - w), wave);
+  return before + x - v;
+}
+
 // Host-side launchers, one per stage file.
 void launchReset(const Params& P, hipStream_t stream);
 void launchFinish(const Params& P, Counters* host, hipStream_t stream);

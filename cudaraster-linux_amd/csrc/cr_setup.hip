@@ -472,24 +472,6 @@ __device__ __forceinline__ uint64_t laneLt() {
   return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
-// Exclusive scan of one value per thread over the whole block (at most 16
-// waves: every wave adds up the wave sums by itself).  One barrier; a scan
-// that may follow without another needs `sums` of its own.
-template <int NT>
-__device__ __forceinline__ uint32_t blockScan(uint32_t v, uint32_t* sums, uint32_t& total) {
-  constexpr int NW = NT / 64;
-  static_assert(NW <= 16, "one row of lanes holds the wave sums");
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t x = waveScan(v);
-  if (lane == 63) sums[wave] = x;
-  __syncthreads();
-  const uint32_t w = lane < NW ? sums[lane] : 0u;
-  const uint32_t sc = waveScan(w);
-  total = (uint32_t)__builtin_amdgcn_readlane((int)sc, NW - 1);
-  const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)(sc - w), wave);
-  return before + x - v;
-}
-
 // Setup and binning of chunk `chunk` of one draw (one 1024-lane workgroup).
 // load(): the draw's parameters; asked for once by the setup and once by the
 // binning, so that a batch, which loads them from its table, need not hold
