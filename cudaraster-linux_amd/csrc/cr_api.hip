@@ -141,9 +141,7 @@ cr_status ensureBuffers(cr_context* ctx, const Geometry& g, int32_t numChunks) {
   CR_HIP(ctx, ctx->triHeader.ensure((size_t)ctx->maxSubtris * sizeof(Header)));
   CR_HIP(ctx, ctx->triData.ensure((size_t)ctx->maxSubtris * sizeof(TriData)));
   CR_HIP(ctx, ctx->subtriTri.ensure((size_t)std::max<int64_t>(ctx->maxSubtris - nt, 1) * 4));
-  CR_HIP(ctx, ctx->chunkBase.ensure((size_t)std::max(numChunks, 1) * 4));
-  CR_HIP(ctx, ctx->binCnt.ensure((size_t)g.nb * std::max(numChunks, 1) * 4));
-  CR_HIP(ctx, ctx->binOff.ensure((size_t)g.nb * std::max(numChunks, 1) * 4));
+  CR_HIP(ctx, ctx->binAddr.ensure((size_t)(g.nb + 1) * std::max(numChunks, 1) * 4));
   CR_HIP(ctx, ctx->binList.ensure((size_t)ctx->maxBinEntries * 16));
   CR_HIP(ctx, ctx->tileStart.ensure((size_t)g.nt * 4));
   CR_HIP(ctx, ctx->tileCount.ensure((size_t)g.nt * 4));
@@ -170,9 +168,7 @@ DrawBuffers contextBuffers(cr_context* ctx) {
   B.triHeader = ctx->triHeader.as<Header>();
   B.triData = ctx->triData.as<TriData>();
   B.subtriTri = ctx->subtriTri.as<uint32_t>();
-  B.chunkBase = ctx->chunkBase.as<uint32_t>();
-  B.binCnt = ctx->binCnt.as<uint32_t>();
-  B.binOff = ctx->binOff.as<uint32_t>();
+  B.binAddr = ctx->binAddr.as<uint32_t>();
   B.binList = ctx->binList.as<uint4>();
   B.tileStart = ctx->tileStart.as<uint32_t>();
   B.tileCount = ctx->tileCount.as<uint32_t>();
@@ -233,9 +229,7 @@ Params makeParams(cr_context* ctx, const Geometry& g, int32_t numChunks, const D
   P.triData = B.triData;
   P.subtriTri = B.subtriTri;
   P.numChunks = numChunks;
-  P.chunkBase = B.chunkBase;
-  P.binCnt = B.binCnt;
-  P.binOff = B.binOff;
+  P.binAddr = B.binAddr;
   P.maxBinEntries = (int32_t)B.maxBinEntries;
   P.binList = B.binList;
   P.tileStart = B.tileStart;
@@ -392,8 +386,7 @@ cr_status cr_context_destroy(cr_context* ctx) {
   if (!ctx) return CR_OK;
   (void)hipSetDevice(ctx->device);
   if (ctx->pending) (void)hipStreamSynchronize(ctx->pendingStream);
-  for (DevBuf* b : {&ctx->triSubtris, &ctx->triHeader, &ctx->triData, &ctx->subtriTri, &ctx->chunkBase,
-                    &ctx->binCnt, &ctx->binOff, &ctx->binList, &ctx->tileStart, &ctx->tileCount,
+  for (DevBuf* b : {&ctx->triSubtris, &ctx->triHeader, &ctx->triData, &ctx->subtriTri, &ctx->binAddr, &ctx->binList, &ctx->tileStart, &ctx->tileCount,
                     &ctx->tileList, &ctx->tileSegNext, &ctx->tileFrags, &ctx->chunkSubtris, &ctx->counters,
                     &ctx->profBuf, &ctx->interpAcc})
     b->release();

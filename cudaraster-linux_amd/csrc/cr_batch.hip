@@ -39,7 +39,7 @@ struct ViewState {
   uint32_t clearColor = 0, clearDepth = 0;
   int64_t maxSubtris = 1, maxBin = 1, maxTile = 1;
   // Element offsets of the view's regions in the shared buffers.
-  size_t oTri = 0, oSlot = 0, oClip = 0, oChunk = 0, oBinCC = 0, oBin = 0, oTile = 0, oTileList = 0;
+  size_t oTri = 0, oSlot = 0, oClip = 0, oBinAddr = 0, oBin = 0, oTile = 0, oTileList = 0;
 };
 
 // One launch set: the device Params table of a list of views and, per
@@ -68,7 +68,7 @@ struct cr_batch {
   cr_context* ctx = nullptr;
   int device = 0;
   std::vector<ViewState> views;
-  DevBuf triSubtris, triHeader, triData, subtriTri, chunkBase, binCnt, binOff, binList;
+  DevBuf triSubtris, triHeader, triData, subtriTri, binAddr, binList;
   DevBuf tileStart, tileCount, tileList, tileSegNext, counters, saved;
   Counters* hostCounters = nullptr;   // pinned, one block per view, written by the draws' finish kernels
   Counters* hostCountersDev = nullptr;   // their device address
@@ -97,7 +97,7 @@ namespace {
 
 cr_status layout(cr_batch* b) {
   cr_context* ctx = b->ctx;
-  size_t nTri = 0, nSlot = 0, nClip = 0, nChunk = 0, nBinCC = 0, nBin = 0, nTile = 0, nTileList = 0;
+  size_t nTri = 0, nSlot = 0, nClip = 0, nBinAddr = 0, nBin = 0, nTile = 0, nTileList = 0;
   for (ViewState& v : b->views) {
     const int64_t nt = v.desc.num_tris;
     v.oTri = nTri;
@@ -106,10 +106,8 @@ cr_status layout(cr_batch* b) {
     nSlot += align64((size_t)v.maxSubtris);
     v.oClip = nClip;
     nClip += align64((size_t)std::max<int64_t>(v.maxSubtris - nt, 1));
-    v.oChunk = nChunk;
-    nChunk += align64((size_t)std::max(v.numChunks, 1));
-    v.oBinCC = nBinCC;
-    nBinCC += align64((size_t)v.g.nb * std::max(v.numChunks, 1));
+    v.oBinAddr = nBinAddr;
+    nBinAddr += align64((size_t)(v.g.nb + 1) * std::max(v.numChunks, 1));
     v.oBin = nBin;
     nBin += align64((size_t)v.maxBin);
     v.oTile = nTile;
@@ -121,9 +119,7 @@ cr_status layout(cr_batch* b) {
   CR_HIP(ctx, b->triHeader.ensure(nSlot * sizeof(Header)));
   CR_HIP(ctx, b->triData.ensure(nSlot * sizeof(TriData)));
   CR_HIP(ctx, b->subtriTri.ensure(nClip * 4));
-  CR_HIP(ctx, b->chunkBase.ensure(nChunk * 4));
-  CR_HIP(ctx, b->binCnt.ensure(nBinCC * 4));
-  CR_HIP(ctx, b->binOff.ensure(nBinCC * 4));
+  CR_HIP(ctx, b->binAddr.ensure(nBinAddr * 4));
   CR_HIP(ctx, b->binList.ensure(nBin * 16));
   CR_HIP(ctx, b->tileStart.ensure(nTile * 4));
   CR_HIP(ctx, b->tileCount.ensure(nTile * 4));
@@ -133,7 +129,7 @@ cr_status layout(cr_batch* b) {
   CR_HIP(ctx, b->counters.ensure(b->views.size() * sizeof(Counters)));
   if (b->counters.ptr != before) b->countersClean = false;
   b->reserved = b->triSubtris.bytes + b->triHeader.bytes + b->triData.bytes + b->subtriTri.bytes +
-                b->chunkBase.bytes + b->binCnt.bytes + b->binOff.bytes + b->binList.bytes + b->tileStart.bytes +
+                b->binAddr.bytes + b->binList.bytes + b->tileStart.bytes +
                 b->tileCount.bytes + b->tileList.bytes + b->tileSegNext.bytes + b->counters.bytes;
   b->graphValid = false;
   b->laidOut = true;
@@ -176,9 +172,7 @@ Params viewParams(const cr_batch* b, int i) {
   P.triData = b->triData.as<TriData>() + v.oSlot;
   P.subtriTri = b->subtriTri.as<uint32_t>() + v.oClip;
   P.numChunks = v.numChunks;
-  P.chunkBase = b->chunkBase.as<uint32_t>() + v.oChunk;
-  P.binCnt = b->binCnt.as<uint32_t>() + v.oBinCC;
-  P.binOff = b->binOff.as<uint32_t>() + v.oBinCC;
+  P.binAddr = b->binAddr.as<uint32_t>() + v.oBinAddr;
   P.maxBinEntries = (int32_t)v.maxBin;
   P.binList = b->binList.as<uint4>() + v.oBin;
   P.tileStart = b->tileStart.as<uint32_t>() + v.oTile;
@@ -237,7 +231,7 @@ cr_status buildTables(cr_batch* b, Tables& T, const std::vector<int>& idx) {
     tileCost[k] = (measured ? (double)c.tileEntries : 2.0 * P.numTris) * (1 << P.samplesLog2) /
                   std::max(P.numTiles, 1);
     chunks[k] = P.numTris > 0 ? P.numChunks : 0;
-    bins[k] = P.numBins;
+    bins[k] = coarseBlocks(P);
     groups[k] = ((P.numTiles + W - 1) / W + kFineRounds - 1) / kFineRounds;
   }
   std::vector<int> all(n);
@@ -559,8 +553,8 @@ cr_status cr_batch_destroy(cr_batch* b) {
   (void)hipDeviceSynchronize();
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
-  for (DevBuf* d : {&b->triSubtris, &b->triHeader, &b->triData, &b->subtriTri, &b->chunkBase, &b->binCnt, &b->binOff,
-                    &b->binList, &b->tileStart, &b->tileCount, &b->tileList, &b->tileSegNext, &b->counters,
+  for (DevBuf* d : {&b->triSubtris, &b->triHeader, &b->triData, &b->subtriTri, &b->binAddr, &b->binList,
+                    &b->tileStart, &b->tileCount, &b->tileList, &b->tileSegNext, &b->counters,
                     &b->saved,
                     &b->subset.params, &b->subset.starts})
     d->release();

@@ -373,7 +373,20 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
   __shared__ uint32_t sProf[8];
 
   if (bin == 0) stampStage(P, kStampCoarse);
-  if (P.counters->overflow & 3u) return;
+  // The overflow flag and the first chunks' counts and addresses of this bin,
+  // issued together: the start waits for one load latency.
+  const uint32_t* row = P.binAddr + bin;
+  const size_t pitch = (size_t)(P.numBins + 1);
+  const int i0 = 2 * threadIdx.x, i1 = i0 + 1;
+  uint32_t n0 = 0, n1 = 0, a0 = 0, a1 = 0;     // chunks i0 and i1: the bin's entries and the first one's address
+  auto loadRow = [&](int cb, int nb) {
+    n0 = n1 = a0 = a1 = 0;
+    if (i0 < nb) { a0 = row[(size_t)(cb + i0) * pitch]; n0 = row[(size_t)(cb + i0) * pitch + 1] - a0; }
+    if (i1 < nb) { a1 = row[(size_t)(cb + i1) * pitch]; n1 = row[(size_t)(cb + i1) * pitch + 1] - a1; }
+  };
+  const uint32_t overflowed = P.counters->overflow;
+  loadRow(0, min(kSegBatch, P.numChunks));
+  if (overflowed & 3u) return;
   const bool prof = P.prof != nullptr;
   if (prof && threadIdx.x < 8) sProf[threadIdx.x] = 0;
   const int bl = P.binLog2, tpb = 1 << (2 * bl);   // tiles per bin side log2, tiles per bin
@@ -381,8 +394,6 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
   // Every tile of the bin's square lies in the viewport.
   const bool binComplete = ((bx + 1) << bl) <= P.widthTiles && ((by + 1) << bl) <= P.heightTiles;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t* bCnt = P.binCnt + (size_t)bin * P.numChunks;
-  const uint32_t* bOff = P.binOff + (size_t)bin * P.numChunks;
   const uint32_t segCap = (uint32_t)P.maxTileEntries >> kTileSegLog2;   // segments the list buffer holds
 
   for (int i = threadIdx.x; i < kBinTiles; i += kCoarseThreads) {
@@ -398,10 +409,9 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
     // Segment table of chunks [cb, cb + nb): start of each segment in the
     // bin's entry order and its address in the bin queue.
     const int nb = min(kSegBatch, P.numChunks - cb);
-    const int i0 = 2 * threadIdx.x, i1 = i0 + 1;
-    const uint32_t n0 = (i0 < nb) ? bCnt[cb + i0] : 0u, n1 = (i1 < nb) ? bCnt[cb + i1] : 0u;
-    if (i0 < nb) segAddr[i0] = P.chunkBase[cb + i0] + bOff[cb + i0];
-    if (i1 < nb) segAddr[i1] = P.chunkBase[cb + i1] + bOff[cb + i1];
+    if (cb > 0) loadRow(cb, nb);
+    if (i0 < nb) segAddr[i0] = a0;
+    if (i1 < nb) segAddr[i1] = a1;
     uint32_t segTotal;
     const uint32_t s0 = blockScan<kCoarseThreads>(n0 + n1, sums, segTotal);
     if (i0 < nb) segStart[i0] = s0;
@@ -652,8 +662,12 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
       P.tileStart[gx + gy * P.widthTiles] = tFirst[threadIdx.x];
       P.tileCount[gx + gy * P.widthTiles] = tTotal[threadIdx.x];
     }
-    if (tTotal[threadIdx.x]) atomicAdd(&sWritten, tTotal[threadIdx.x]);
   }
+  const uint32_t written =
+      (uint32_t)waveReduce(threadIdx.x < (unsigned)tpb ? (int32_t)tTotal[threadIdx.x] : 0, 0,
+                           [](int32_t a, int32_t b) { return a + b; });
+  // (One device atomic per bin: those of one address take about 5 ns each.)
+  if (lane == 0 && written) atomicAdd(&sWritten, written);
   __syncthreads();
   if (threadIdx.x == 0 && sWritten) atomicAdd(&P.counters->tileListEntries, sWritten);
   if (prof && threadIdx.x == 0) {
@@ -671,14 +685,19 @@ __device__ __forceinline__ void coarseBody(const Params& P, const int bin) {
   }
 }
 
+// XCD-aware order: workgroup b runs on XCD b % 8, so each XCD gets one
+// contiguous band of a view's bins (coarseBlocks() workgroups, a multiple of
+// 8).  Neighbouring bins' runs of a chunk share the bin queue's and the
+// address rows' cache lines, which are then read into one L2 instead of
+// several.
+__device__ __forceinline__ int coarseBin(const Params& P, int block) {
+  const int per = (P.numBins + 7) >> 3;
+  return (block & 7) * per + (block >> 3);
+}
+
 template <int CT>
 __global__ void __launch_bounds__(CT) coarseKernel(const Params P) {
-  // XCD-aware order: workgroup b runs on XCD b % 8, so each XCD gets one
-  // contiguous band of bins.  Neighbouring bins' runs of a chunk share the
-  // bin queue's cache lines, which are then read into one L2 instead of
-  // several.
-  const int per = (P.numBins + 7) >> 3;
-  const int bin = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  const int bin = coarseBin(P, (int)blockIdx.x);
   if (bin >= P.numBins) return;
   coarseBody<CT>(P, bin);
 }
@@ -689,7 +708,9 @@ __global__ void __launch_bounds__(CT) coarseBatchKernel(const Params* __restrict
                                                         const int32_t* __restrict__ order, int numViews) {
   const int k = findView(blockStart, numViews, (int)blockIdx.x);
   const Params P = loadParams(&views[order[k]]);
-  coarseBody<CT>(P, (int)blockIdx.x - blockStart[k]);
+  const int bin = coarseBin(P, (int)blockIdx.x - blockStart[k]);
+  if (bin >= P.numBins) return;
+  coarseBody<CT>(P, bin);
 }
 
 // One workgroup per view: clears the view's counter block.
@@ -715,17 +736,22 @@ void launchFinishBatch(const Params* views, int numViews, const Counters* devBas
 
 int coarseShapeFor(const Params& P) {
   if (P.coarseThreads == 256 || P.coarseThreads == 1024) return P.coarseThreads;
-  // A single draw leaves the GPU room for the large workgroups (measured
-  // faster from 32k triangles at 256^2 to 1M at 2048^2); the small ones pay
-  // off when many draws share the GPU (batches tune it).
+  // A single draw leaves the GPU room for the large workgroups, which hide
+  // more of a long bin's latency (100k triangles at 1024^2 14.1 against 17.4
+  // us, 1M at 2048^2 37 against 72); with few entries per bin there is nothing
+  // to hide and the small ones' barriers are cheaper (12 triangles 12.0 against
+  // 10.9 us, 30k 13.1 against 12.2).  Batches tune it.
+  if (P.numTris < 32 * 1024) return 256;
   return 1024;
 }
 
+int coarseBlocks(const Params& P) { return ((P.numBins + 7) >> 3) * 8; }
+
 void launchCoarse(const Params& P, hipStream_t stream) {
   if (coarseShapeFor(P) == 1024)
-    hipLaunchKernelGGL(coarseKernel<1024>, dim3(((P.numBins + 7) >> 3) * 8), dim3(1024), 0, stream, P);
+    hipLaunchKernelGGL(coarseKernel<1024>, dim3(coarseBlocks(P)), dim3(1024), 0, stream, P);
   else
-    hipLaunchKernelGGL(coarseKernel<256>, dim3(((P.numBins + 7) >> 3) * 8), dim3(256), 0, stream, P);
+    hipLaunchKernelGGL(coarseKernel<256>, dim3(coarseBlocks(P)), dim3(256), 0, stream, P);
 }
 
 // Points views [first, first + n) at other vertex and index buffers.

@@ -172,13 +172,12 @@ struct Params {
   Header* triHeader;
   TriData* triData;
   uint32_t* subtriTri;             // source triangle of slots >= numTris
-  // Bin queue: chunk c (kSetupChunkTris triangles) owns a region starting at
-  // chunkBase[c]; bin b's entries of chunk c are binCnt[b][c] slots at
-  // region offset binOff[b][c], in submission order.
+  // Bin queue: chunk c (kSetupChunkTris triangles) owns a region of it, in
+  // which bin b's entries, in submission order, are binList[binAddr[c][b]] to
+  // binList[binAddr[c][b + 1] - 1].  Chunk-major: a setup workgroup writes its
+  // row in one piece, and the bins of an XCD's band read the same lines.
   int32_t numChunks;
-  uint32_t* chunkBase;             // [numChunks]
-  uint32_t* binCnt;                // [numBins][numChunks]
-  uint32_t* binOff;                // [numBins][numChunks]
+  uint32_t* binAddr;               // [numChunks][numBins + 1]
   int32_t maxBinEntries;
   uint4* binList;                  // per entry: slot, then the header's three snapped vertices
   // Tile lists in submission order, each a chain of kTileSeg-entry
@@ -342,9 +341,7 @@ __device__ __forceinline__ Params loadParams(const Params* view) {
   makeGlobal(P.triHeader);
   makeGlobal(P.triData);
   makeGlobal(P.subtriTri);
-  makeGlobal(P.chunkBase);
-  makeGlobal(P.binCnt);
-  makeGlobal(P.binOff);
+  makeGlobal(P.binAddr);
   makeGlobal(P.binList);
   makeGlobal(P.tileStart);
   makeGlobal(P.tileCount);
@@ -434,6 +431,7 @@ void launchCoarseBatch(int threads, const Params* views, const int32_t* blockSta
                        int numViews, int totalBlocks, hipStream_t stream);
 constexpr int kCoarseShapes[2] = {256, 1024};    // coarse workgroup sizes (lanes) compiled
 int coarseShapeFor(const Params& P);             // the plain draw's choice
+int coarseBlocks(const Params& P);               // workgroups of a draw's (or view's) coarse stage
 // Fine-stage variant of a draw: (samplesLog2 * 2 + deferred shading) * 2 + depth test.
 constexpr int kFineVariants = 16;
 // Tile groups per workgroup of a batched fine pass: the workgroup walks them

@@ -113,9 +113,7 @@ struct DrawBuffers {
   crhip::Header* triHeader = nullptr;
   crhip::TriData* triData = nullptr;
   uint32_t* subtriTri = nullptr;
-  uint32_t* chunkBase = nullptr;
-  uint32_t* binCnt = nullptr;
-  uint32_t* binOff = nullptr;
+  uint32_t* binAddr = nullptr;        // numChunks rows of numBins + 1
   uint4* binList = nullptr;
   uint32_t* tileStart = nullptr;
   uint32_t* tileCount = nullptr;
@@ -178,7 +176,7 @@ struct cr_context {
 
   int64_t maxSubtris = 1, maxBinEntries = 1, maxTileEntries = 1;
   crhost::DevBuf triSubtris, triHeader, triData, subtriTri;
-  crhost::DevBuf chunkBase, binCnt, binOff, binList;
+  crhost::DevBuf binAddr, binList;
   crhost::DevBuf tileStart, tileCount, tileList, tileSegNext, tileFrags, chunkSubtris;
   crhost::DevBuf counters, profBuf;
   crhost::DevBuf interpAcc;                  // fixed-point gradient accumulators (deterministic backward)

@@ -55,8 +55,7 @@ size_t fixedBytes(int64_t numTris, const crhost::Geometry& g, int32_t numChunks,
   const size_t nc = (size_t)std::max(numChunks, 1);
   size_t b = alignUp(sizeof(Counters));
   b += alignUp((size_t)std::max<int64_t>(numTris, 1));      // triSubtris
-  b += alignUp(nc * 4);                                       // chunkBase
-  b += 2 * alignUp((size_t)g.nb * nc * 4);                    // binCnt, binOff
+  b += alignUp((size_t)(g.nb + 1) * nc * 4);                  // binAddr
   b += 2 * alignUp((size_t)g.nt * 4);                         // tileStart, tileCount
   if (counting) b += alignUp((size_t)g.nt * 4) + alignUp(nc * 4);   // tileFrags, chunkSubtris
   if (profiling) b += alignUp(2 * kProfCount * sizeof(unsigned long long));
@@ -86,9 +85,7 @@ crhost::DrawBuffers layout(uint8_t* base, int64_t numTris, const crhost::Geometr
   B.maxTileEntries = tile;
   B.counters = reinterpret_cast<Counters*>(take(sizeof(Counters)));
   B.triSubtris = take((size_t)std::max<int64_t>(numTris, 1));
-  B.chunkBase = reinterpret_cast<uint32_t*>(take(nc * 4));
-  B.binCnt = reinterpret_cast<uint32_t*>(take((size_t)g.nb * nc * 4));
-  B.binOff = reinterpret_cast<uint32_t*>(take((size_t)g.nb * nc * 4));
+  B.binAddr = reinterpret_cast<uint32_t*>(take((size_t)(g.nb + 1) * nc * 4));
   B.tileStart = reinterpret_cast<uint32_t*>(take((size_t)g.nt * 4));
   B.tileCount = reinterpret_cast<uint32_t*>(take((size_t)g.nt * 4));
   if (counting) {

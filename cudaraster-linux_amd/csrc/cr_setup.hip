@@ -613,7 +613,7 @@ __device__ __forceinline__ void setupBinBody(Load&& load, const int chunk) {
     __syncthreads();
   }
 
-  // ---- reserve the chunk's region; publish counts and offsets ---------------
+  // ---- reserve the chunk's region; publish the bins' addresses --------------
   uint32_t tot2;
   const uint32_t c = (threadIdx.x < (unsigned)P.numBins) ? cnt[threadIdx.x] : 0u;
   const uint32_t off = blockScan<kSetupChunk>(c, sums[1], tot2);
@@ -629,15 +629,14 @@ __device__ __forceinline__ void setupBinBody(Load&& load, const int chunk) {
       b = 0xFFFFFFFFu;
     }
     sBase = b;
-    P.chunkBase[chunk] = b;
   }
-  if (threadIdx.x < (unsigned)P.numBins) {
-    P.binCnt[(size_t)threadIdx.x * P.numChunks + chunk] = c;
-    P.binOff[(size_t)threadIdx.x * P.numChunks + chunk] = off;
-    run[threadIdx.x] = off;
-  }
+  if (threadIdx.x < (unsigned)P.numBins) run[threadIdx.x] = off;
   __syncthreads();
   const uint32_t regionBase = sBase;
+  // (Where the queue overflowed the row is never read.)
+  uint32_t* row = P.binAddr + (size_t)chunk * (size_t)(P.numBins + 1);
+  if (threadIdx.x < (unsigned)P.numBins) row[threadIdx.x] = regionBase + off;
+  if (threadIdx.x == 0) row[P.numBins] = regionBase + tot2;
   if (regionBase == 0xFFFFFFFFu || tot2 == 0) return;
 
   // ---- pass 2: write the entries in order ------------------------------------
