@@ -177,7 +177,7 @@ DrawBuffers contextBuffers(cr_context* ctx) {
   B.tileFrags = countingDraw(ctx) ? ctx->tileFrags.as<uint32_t>() : nullptr;
   B.chunkSubtris = countingDraw(ctx) ? ctx->chunkSubtris.as<uint32_t>() : nullptr;
   B.prof = profilingDraw(ctx) ? ctx->profBuf.as<unsigned long long>() : nullptr;
-  B.counters = ctx->counters.as<Counters>();
+  B.counters = ctx->counters.as<Counters>() + ctx->counterBlock;
   return B;
 }
 
@@ -244,24 +244,35 @@ Params makeParams(cr_context* ctx, const Geometry& g, int32_t numChunks, const D
   return P;
 }
 
-cr_status launchAll(cr_context* ctx, const Params& P, hipStream_t stream, bool reset) {
+cr_status launchAll(cr_context* ctx, Params P, hipStream_t stream, bool own) {
   // A captured draw runs when its graph is launched, after whatever other
-  // draws: it clears the block itself and says nothing about its state now.
+  // draws: it has a block of its own, clears it itself and says nothing about
+  // the others' state now.
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
     (void)hipGetLastError();
     cap = hipStreamCaptureStatusNone;
   }
-  const bool captured = cap != hipStreamCaptureStatusNone;
-  if (reset || captured || !ctx->countersClean || P.prof) launchReset(P, stream);
-  if (!captured && !reset) ctx->countersClean = false;
+  if (cap != hipStreamCaptureStatusNone && own) {
+    own = false;
+    P.counters = ctx->counters.as<Counters>() + 2;
+  }
+  const bool finish = !own || countingDraw(ctx);
+  if (!own || !ctx->countersClean || P.prof) launchReset(P, stream);
+  if (own) ctx->countersClean = false;
+  if (!finish) {
+    P.hostCounters = ctx->hostCountersDev;
+    P.nextCounters = ctx->counters.as<Counters>() + (ctx->counterBlock ^ 1);
+  }
   launchSetup(P, stream);                       // setup and binning are one kernel
   launchCoarse(P, stream);
   launchFine(P, stream);
   launchFragmentSum(P, stream);
-  launchFinish(P, ctx->hostCountersDev, stream);
+  if (finish) launchFinish(P, ctx->hostCountersDev, stream);
   CR_HIP(ctx, hipGetLastError());
-  if (!captured && !reset) ctx->countersClean = true;
+  if (own) ctx->countersClean = true;
+  if (!finish) ctx->counterBlock ^= 1;
+  ctx->lastEnd = finish ? nullptr : P.counters;
   if (P.prof)
     CR_HIP(ctx, hipMemcpyAsync(ctx->hostProf, P.prof, 2 * kProfCount * sizeof(unsigned long long),
                                hipMemcpyDeviceToHost, stream));
@@ -324,7 +335,7 @@ cr_status drawImpl(cr_context* ctx, hipStream_t stream, bool sync) {
     st = ensureBuffers(ctx, g, numChunks);
     if (st != CR_OK) return st;
     Params P = makeParams(ctx, g, numChunks, contextBuffers(ctx));
-    st = launchAll(ctx, P, stream, false);
+    st = launchAll(ctx, P, stream, true);
     if (st != CR_OK) return st;
     if (!sync) {
       // Waiting on this event (not on the stream) lets cr_draw_check return
@@ -366,7 +377,7 @@ cr_status cr_context_create(cr_context** out) {
   // The no-allocation draw's scratch array on this device (looked up once;
   // a failed lookup is reported by that entry point, not here).
   if (e == hipSuccess) scratchInit(ctx->device);
-  if (e == hipSuccess) e = ctx->counters.ensure(sizeof(Counters));
+  if (e == hipSuccess) e = ctx->counters.ensure(3 * sizeof(Counters));
   if (e == hipSuccess) e = hipHostMalloc((void**)&ctx->hostCounters, sizeof(Counters), hipHostMallocDefault);
   if (e == hipSuccess)
     e = hipHostMalloc((void**)&ctx->hostProf, 2 * kProfCount * sizeof(unsigned long long), hipHostMallocDefault);
@@ -612,7 +623,16 @@ cr_status cr_get_stats(cr_context* ctx, cr_stats* out) {
   // Each stage lasts until the next one starts.  Binning runs inside the
   // setup kernel: its time is part of setup_time and bin_time is 0.  (A draw
   // without triangles has no setup stage and no setup stamp.)
-  const uint64_t* s = ctx->hostCounters->stamp;
+  uint64_t s[kStampCount];
+  memcpy(s, ctx->hostCounters->stamp, sizeof(s));
+  if (ctx->lastEnd) {
+    // The fine stage's workgroups left their ends in the device's block, which
+    // the next draw clears (a copy per request, not per draw).
+    Counters c;
+    CR_HIP(ctx, hipSetDevice(ctx->device));
+    CR_HIP(ctx, hipMemcpy(&c, ctx->lastEnd, sizeof(c), hipMemcpyDeviceToHost));
+    s[kStampEnd] = *std::max_element(c.fineEnd, c.fineEnd + 8);
+  }
   const double tick = clockTick(ctx->device);
   auto seconds = [&](uint64_t from, uint64_t to) {
     return from != 0 && to > from ? (float)((double)(to - from) * tick) : 0.0f;

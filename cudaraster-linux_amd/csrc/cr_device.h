@@ -75,8 +75,12 @@ static_assert(sizeof(TriData) == 64, "data layout");
 // kernel and a counter copy, 55 us without (1M triangles: 324 -> 307 us).
 enum Stamp : int { kStampSetup = 0, kStampCoarse, kStampFine, kStampEnd, kStampCount };
 
-// Device counters; one 256-byte block per context.  All zero between draws:
-// the finish kernel hands them to the host and clears them.
+// Device counters, 256 bytes.  All zero before a draw.  A plain draw's context
+// has two blocks that its draws use in turn: the counters are final when the
+// fine stage starts, so its first workgroup hands them to the host, and clears
+// the block of the draw before, which the next one will use.  Draws that count
+// more afterwards, captured draws and batches end with a finish kernel that
+// does both for their own block (3.5 us and a launch gap).
 struct Counters {
   uint32_t numSubtris;     // clipped subtriangles' slots in use past numTris (host copy: plus numTris)
   uint32_t tileEntries;    // tile-list allocator: entries reserved, in whole 32-entry segments
@@ -87,7 +91,8 @@ struct Counters {
   uint64_t fragments;      // (subtriangle, pixel) pairs with >= 1 covered sample
   uint64_t visibleSubtris; // subtriangles that survive setup (counting draws only)
   uint64_t stamp[kStampCount];   // wall clock at the stages' starts and the draw's end (0: stage not run)
-  uint64_t pad[26 - kStampCount];
+  uint64_t fineEnd[8];           // per XCD: wall clock at a last fine workgroup's end (draws without a finish kernel)
+  uint64_t pad[26 - kStampCount - 8];
 };
 static_assert(sizeof(Counters) == 256, "counter block");
 
@@ -195,6 +200,8 @@ struct Params {
   uint32_t* depth;
   uint32_t* triid;                 // optional
   Counters* counters;
+  Counters* hostCounters;          // the fine stage hands the counters over to these (null: a finish kernel does)
+  Counters* nextCounters;          // and clears these (null: none)
 };
 
 // ---------------------------------------------------------------------------
@@ -351,6 +358,7 @@ __device__ __forceinline__ Params loadParams(const Params* view) {
   makeGlobal(P.depth);
   makeGlobal(P.triid);
   makeGlobal(P.counters);
+  P.hostCounters = P.nextCounters = nullptr;   // (a batch ends with a finish kernel)
   return P;
 }
 

@@ -23,6 +23,7 @@
 //    deferred: the loop records (subtriangle slot, centroid) per sample and
 //    the tile is shaded once per (pixel, distinct triangle) at the end.
 //    SrcOver and Additive blend in submission order inside the loop.
+#include <cstddef>
 #include <utility>
 
 #include "cr_device.h"
@@ -255,6 +256,35 @@ __device__ __forceinline__ void waveSync() {
 __device__ __forceinline__ int xcdGroup(int groups) {
   const int per = (groups + 7) >> 3;
   return (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+}
+
+// A plain draw's end, by workgroups of the fine stage themselves: the first
+// one hands the counters to the host (pinned memory, visible when the kernel
+// has ended) and clears the next draw's; each notes its end.
+__device__ __forceinline__ void handOver(const Params& P, int group) {
+  static_assert(sizeof(Counters) == 64 * 4, "one word per lane");
+  if (group != 0 || P.hostCounters == nullptr || threadIdx.x >= 64) return;
+  const int i = (int)threadIdx.x;
+  uint32_t v = reinterpret_cast<const uint32_t*>(P.counters)[i];
+  constexpr int kStart = (int)(offsetof(Counters, stamp) / 4) + 2 * kStampFine;
+  const uint64_t now = wall_clock64();
+  if (i == (int)(offsetof(Counters, numSubtris) / 4)) v += (uint32_t)P.numTris;
+  if (i == kStart) v = (uint32_t)now;
+  if (i == kStart + 1) v = (uint32_t)(now >> 32);
+  reinterpret_cast<uint32_t*>(P.hostCounters)[i] = v;
+  if (P.nextCounters != nullptr) reinterpret_cast<uint32_t*>(P.nextCounters)[i] = 0;
+}
+// (Called by kernels whose first argument is the draw's Params; it reads the
+// two pointers there again, so that nothing is kept in registers for it.)
+__device__ __forceinline__ void noteEnd() {
+  using Arg = const __attribute__((address_space(4))) uint8_t;
+  Arg* args = (Arg*)__builtin_amdgcn_kernarg_segment_ptr();
+  __asm__ volatile("" : "+s"(args));
+  using Word = const __attribute__((address_space(4))) uint64_t;
+  if (*(Word*)(args + offsetof(Params, hostCounters)) == 0 || threadIdx.x != 0) return;
+  Counters* c = (Counters*)(uintptr_t)*(Word*)(args + offsetof(Params, counters));
+  makeGlobal(c);
+  c->fineEnd[blockIdx.x & 7] = wall_clock64();
 }
 
 // Waves per SIMD the 1x-4x deferred-shading copies are held to (at most
@@ -840,7 +870,9 @@ __global__ void __launch_bounds__(64 * kFineWaves, (fineMinWaves<S, VIS>())) fin
   const int groups = (P.numTiles + kFineWaves - 1) / kFineWaves;
   const int group = xcdGroup(groups);
   if (group >= groups) return;
+  if (!COUNT) handOver(P, group);
   fineDispatch<S, VIS, COUNT, kFineWaves, DEPTH>(P, group, recAll);
+  if (!COUNT) noteEnd();
 }
 
 // The texPhong shader: in-order shading with the shader compiled in, blend
@@ -851,7 +883,9 @@ __global__ void __launch_bounds__(64 * kFineWaves) fineTexKernel(const Params P)
   const int groups = (P.numTiles + kFineWaves - 1) / kFineWaves;
   const int group = xcdGroup(groups);
   if (group >= groups) return;
+  if (!COUNT) handOver(P, group);
   fineBody<S, false, COUNT, kFineWaves, DEPTH, -1, true>(P, group, recAll);
+  if (!COUNT) noteEnd();
 }
 
 template <int S, bool COUNT, bool DEPTH>

@@ -136,10 +136,11 @@ cr_status validateDraw(cr_context* ctx);
 DrawBuffers contextBuffers(cr_context* ctx);
 // Kernel parameters of the context's current state over buffers B.
 crhip::Params makeParams(cr_context* ctx, const Geometry& g, int32_t numChunks, const DrawBuffers& B);
-// Setup+bin, coarse, fine and finish launches on `stream`; the last one puts
-// the counters into ctx->hostCounters and clears the block.  reset: clear the
-// block before the draw too (a block that other draws may have left in use).
-cr_status launchAll(cr_context* ctx, const crhip::Params& P, hipStream_t stream, bool reset);
+// Setup+bin, coarse, fine and, where the fine stage does not do its work
+// itself, finish launches on `stream`: the counters end up in
+// ctx->hostCounters.  own: P.counters is the context's block of its next draw;
+// else a block that other draws may have left in use, cleared first.
+cr_status launchAll(cr_context* ctx, crhip::Params P, hipStream_t stream, bool own);
 // Copies the read-back counters into ctx->last; returns their overflow bits.
 uint32_t recordCounters(cr_context* ctx);
 // Looks up this device's copy of the no-allocation draw's fixed scratch
@@ -178,15 +179,17 @@ struct cr_context {
   crhost::DevBuf triSubtris, triHeader, triData, subtriTri;
   crhost::DevBuf binAddr, binList;
   crhost::DevBuf tileStart, tileCount, tileList, tileSegNext, tileFrags, chunkSubtris;
-  crhost::DevBuf counters, profBuf;
+  crhost::DevBuf counters, profBuf;          // counters: two blocks for draws in turn, one for captured draws
   crhost::DevBuf interpAcc;                  // fixed-point gradient accumulators (deterministic backward)
   crhip::Counters* hostCounters = nullptr;   // pinned, written by the draw's finish kernel
   crhip::Counters* hostCountersDev = nullptr;   // its device address
-  bool countersClean = false;                // the last draw of `counters` was queued whole: it leaves them cleared
+  bool countersClean = false;                // the last draw was queued whole: it leaves the next block cleared
+  int counterBlock = 0;                      // which of the two blocks in `counters` the next draw uses
+  const crhip::Counters* lastEnd = nullptr;  // the last draw's device block when it holds the end stamps
   unsigned long long* hostProf = nullptr;    // pinned, 2 * kProfCount
   cr_profile_counters lastProf{};
   bool lastProfiled = false;                 // the last launch recorded profile counters
-  bool drawn = false;                 // hostCounters hold (or will hold) a draw's stamps
+  bool drawn = false;                 // hostCounters hold (or will hold) a draw's counters and stamps
   hipStream_t pendingStream = nullptr;
   hipEvent_t evPending = nullptr;     // after an asynchronous draw's counter readback
   bool pending = false;

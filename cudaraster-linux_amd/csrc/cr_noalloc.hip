@@ -208,7 +208,7 @@ extern "C" cr_status cr_draw_triangles_noalloc(cr_context* ctx, void* stream) {
     const DrawBuffers B =
         layout(static_cast<uint8_t*>(base), nt, g, numChunks, counting, profiling, subtris, bin, tile);
     const Params P = makeParams(ctx, g, numChunks, B);
-    st = launchAll(ctx, P, s, true);        // the array's counter block is shared by every context
+    st = launchAll(ctx, P, s, false);       // the array's counter block is shared by every context
     if (st != CR_OK) return st;
     CR_HIP(ctx, hipStreamSynchronize(s));
     const uint32_t ov = recordCounters(ctx);
