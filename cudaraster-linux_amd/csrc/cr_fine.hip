@@ -736,12 +736,11 @@ __device__ __forceinline__ void fineBody(const Params& P, const int group, uint3
             const uint32_t tri = triWord & 0x7FFFFFFFu;
             bool discard = false;
             if (TEX) {
-              if (anyWr) {
-                const uint32_t* q = r + L::SH;
-                const Planes pl = {(int32_t)q[0], (int32_t)q[1], (int32_t)q[2], (int32_t)q[3], (int32_t)q[4],
-                                   (int32_t)q[5], (int32_t)q[6], (int32_t)q[7], (int32_t)q[8]};
-                discard = shadeTexPhong<S>(P, pl, q[9], q[10], q[11], tri, code, px, py, &src);
-              }
+              const uint32_t* q = r + L::SH;
+              auto word = [&](int k) { return __builtin_amdgcn_readfirstlane((int)q[k]); };   // (one record per wave)
+              const Planes pl = {word(0), word(1), word(2), word(3), word(4), word(5), word(6), word(7), word(8)};
+              const uint32_t v0 = (uint32_t)word(9), v1 = (uint32_t)word(10), v2 = (uint32_t)word(11);
+              if (anyWr) discard = shadeTexPhong<S>(P, pl, v0, v1, v2, tri, code, px, py, &src);
             } else if (anyWr && gouraud) {
               const uint32_t* q = r + L::SH;
               const uint4 t1 = make_uint4(q[0], q[1], q[2], q[3]);
@@ -876,9 +875,12 @@ __global__ void __launch_bounds__(64 * kFineWaves, (fineMinWaves<S, VIS>())) fin
 }
 
 // The texPhong shader: in-order shading with the shader compiled in, blend
-// mode from the draw.
+// mode from the draw.  Bound by VALU issue with too few waves to hide the
+// texture fetches: 20k triangles of 4-3000 pixels, 1024x768 4x, quads, 152 us
+// at three waves per SIMD with per-lane copies of what is uniform, 116 us with
+// it in scalar registers and five waves (four at 8x, where five would spill).
 template <int S, bool COUNT, bool DEPTH>
-__global__ void __launch_bounds__(64 * kFineWaves) fineTexKernel(const Params P) {
+__global__ void __launch_bounds__(64 * kFineWaves, S <= 2 ? 5 : 4) fineTexKernel(const Params P) {
   __shared__ __attribute__((aligned(16))) uint32_t recAll[kFineWaves * recWords<S, false>()];
   const int groups = (P.numTiles + kFineWaves - 1) / kFineWaves;
   const int group = xcdGroup(groups);

@@ -20,6 +20,16 @@
 
 namespace crhip {
 
+// Loads of what is the same for the whole wave (a record's vertices and
+// material) and not written by the kernel: through the scalar path, into
+// scalar registers.  As vector loads the nine varyings alone took 36 registers
+// of every lane (fine pass of 20k triangles, 1024x768 4x: 152 -> 122 us).
+template <class T>
+__device__ __forceinline__ T uniformLoad(const void* p) {
+  return *(const __attribute__((address_space(4))) T*)(uintptr_t)p;
+}
+typedef float crFloatx4 __attribute__((ext_vector_type(4)));
+
 // log2: x = m 2^e, m in [sqrt(1/2), sqrt(2)); ln m = 2 atanh(t),
 // t = (m-1)/(m+1), atanh t = t (1 + t^2/3 + t^4/5 + t^6/7 + t^8/9).
 __device__ __forceinline__ float crLog2(float x) {
@@ -71,11 +81,14 @@ __device__ __forceinline__ float crPow(float x, float y) {
 }
 
 // Texel index of floor value f wrapped into [0, n); NaN and out-of-range
-// values give 0.
+// values give 0.  Coordinates are mostly within one texture of [0, n), where
+// an addition does it; the division costs some forty instructions.
 __device__ __forceinline__ int32_t wrapIndex(float f, int32_t n) {
+  const int32_t k = (int32_t)f;
+  if (fabsf(f) < 16384.0f && k >= -n && k < 2 * n) return k < 0 ? k + n : k >= n ? k - n : k;
   if (!(fabsf(f) < 1073741824.0f)) return 0;
-  const int32_t k = (int32_t)f % n;
-  return k < 0 ? k + n : k;
+  const int32_t m = k % n;
+  return m < 0 ? m + n : m;
 }
 
 // tex2D on the float4 atlas: normalised (u, v), wrap addressing, bilinear in
@@ -101,8 +114,9 @@ __device__ __forceinline__ float4 texSample(const float4* __restrict__ atlas, in
 // texture2D (Shaders.cu:125-148).
 __device__ __forceinline__ float4 texture2D(const TexSpec& spec, const float4* __restrict__ atlas, int32_t w,
                                             int32_t h, float2 tex, float2 texDX, float2 texDY) {
-  const float ax = texDX.x * spec.size[0], ay = texDX.y * spec.size[1];
-  const float bx = texDY.x * spec.size[0], by = texDY.y * spec.size[1];
+  const float sizeX = uniformLoad<float>(&spec.size[0]), sizeY = uniformLoad<float>(&spec.size[1]);
+  const float ax = texDX.x * sizeX, ay = texDX.y * sizeY;
+  const float bx = texDY.x * sizeX, by = texDY.y * sizeY;
   const float dxlen = fmaf(ax, ax, ay * ay);
   const float dylen = fmaf(bx, bx, by * by);
   const float lod = fminf(fmaxf(crLog2(fmaxf(dxlen, dylen)) * 0.5f, 0.0f), 14.0f);
@@ -136,10 +150,10 @@ __device__ __forceinline__ float3 evaluateLighting(float3 cameraPos, float3 came
   const float s2 = dotIN * 2.0f;
   const float3 R = make_float3(fmaf(-N.x, s2, I.x), fmaf(-N.y, s2, I.y), fmaf(-N.z, s2, I.z));
   const float diffuseCoef = fmaf(fmaxf(-dotIN, 0.0f), 0.75f, 0.25f);
-  const float specularCoef = crPow(fmaxf(-dot3(I, R), 0.0f), m.glossiness);
-  return make_float3(fmaf(diffuseCoef, diffuse.x, specularCoef * m.specular[0]),
-                     fmaf(diffuseCoef, diffuse.y, specularCoef * m.specular[1]),
-                     fmaf(diffuseCoef, diffuse.z, specularCoef * m.specular[2]));
+  const float specularCoef = crPow(fmaxf(-dot3(I, R), 0.0f), uniformLoad<float>(&m.glossiness));
+  return make_float3(fmaf(diffuseCoef, diffuse.x, specularCoef * uniformLoad<float>(&m.specular[0])),
+                     fmaf(diffuseCoef, diffuse.y, specularCoef * uniformLoad<float>(&m.specular[1])),
+                     fmaf(diffuseCoef, diffuse.z, specularCoef * uniformLoad<float>(&m.specular[2])));
 }
 
 // Barycentric planes of one subtriangle (TriData words 4..12).
@@ -175,7 +189,8 @@ __device__ __forceinline__ float4 interpVarying(const float4& c0, const float4& 
 }
 
 __device__ __forceinline__ float4 loadVarying(const uint8_t* verts, uint32_t vi, int stride, int k) {
-  return *reinterpret_cast<const float4*>(verts + (uint64_t)vi * (uint32_t)stride + 16 + 16 * k);
+  const crFloatx4 v = uniformLoad<crFloatx4>(verts + (uint64_t)vi * (uint32_t)stride + 16 + 16 * k);
+  return make_float4(v.x, v.y, v.z, v.w);
 }
 
 // Texture coordinate (varying 2) at the centre of pixel (px, py).
@@ -190,9 +205,10 @@ __device__ __forceinline__ float2 centerTex(const Planes& q, int px, int py, con
 }
 
 // FragmentShader_texPhong::run for pixel (px, py) of source triangle tri,
-// coverage centroid code (15: pixel centre).  Returns true when the
-// fragment is discarded (alpha test, or a material index outside the
-// table); otherwise *color is the shaded ABGR colour.
+// coverage centroid code (15: pixel centre).  The triangle (planes, vertex
+// indices, tri) is the same in every lane and in scalar registers.  Returns
+// true when the fragment is discarded (alpha test, or a material index outside
+// the table); otherwise *color is the shaded ABGR colour.
 template <int S>
 __device__ __forceinline__ bool shadeTexPhong(const Params& P, const Planes& q, uint32_t vi0, uint32_t vi1,
                                               uint32_t vi2, uint32_t tri, int code, int px, int py,
@@ -241,17 +257,18 @@ __device__ __forceinline__ bool shadeTexPhong(const Params& P, const Planes& q, 
     texDX = oddX ? make_float2(tex.x - ox.x, tex.y - ox.y) : make_float2(ox.x - tex.x, ox.y - tex.y);
     texDY = oddY ? make_float2(tex.x - oy.x, tex.y - oy.y) : make_float2(oy.x - tex.x, oy.y - tex.y);
   }
-  const int32_t mi = (int64_t)tri < P.numTriMaterials ? P.triMaterial[tri] : -1;
+  const int32_t mi = (int64_t)tri < P.numTriMaterials ? uniformLoad<int32_t>(P.triMaterial + tri) : -1;
   if (mi < 0 || mi >= P.numMaterials) return true;
   const Material& M = P.materials[mi];
-  float4 dc = M.diffuse;
-  if (M.diffuseTexture.size[0] != 0.0f) {
+  const crFloatx4 diffuse = uniformLoad<crFloatx4>(&M.diffuse);
+  float4 dc = make_float4(diffuse.x, diffuse.y, diffuse.z, diffuse.w);
+  if (uniformLoad<float>(&M.diffuseTexture.size[0]) != 0.0f) {
     const float4 t = texture2D(M.diffuseTexture, P.atlas, P.atlasWidth, P.atlasHeight, tex, texDX, texDY);
     dc.x = t.x;
     dc.y = t.y;
     dc.z = t.z;
   }
-  if (M.alphaTexture.size[0] != 0.0f)
+  if (uniformLoad<float>(&M.alphaTexture.size[0]) != 0.0f)
     dc.w = texture2D(M.alphaTexture, P.atlas, P.atlasWidth, P.atlasHeight, tex, texDX, texDY).y;
   if (dc.w < 0.5f) return true;
   const float3 c = evaluateLighting(make_float3(cp.x, cp.y, cp.z), make_float3(cn.x, cn.y, cn.z), M,
