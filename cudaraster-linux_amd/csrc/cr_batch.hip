@@ -7,8 +7,8 @@
 // keeps a device table of per-view Params, and runs each stage as one grid
 // over the work of every view: setup+bin over all triangle chunks, coarse
 // over all bins, fine over all tile groups of each pipe variant (the
-// workgroup -> view lookup is a binary search over a prefix table).  The
-// launch sequence is captured once in a hipGraph and replayed.
+// workgroup -> view lookup is a binary search over a prefix table).  From the
+// second draw on the launch sequence is replayed from a captured hipGraph.
 //
 // Per view the kernels are the plain draw's, with the same Params, so every
 // image is bit-identical to a plain draw of that view.  Overflow is per view:
@@ -49,6 +49,7 @@ struct Tables {
     int variant = -1;          // fine stages: pipe variant
     int n = 0;                 // listed views
     int blocks = 0;            // workgroups (fine: tile groups)
+    int64_t tiles = 0;         // fine stages: tiles of the listed views
     int ofs = 0, orderOfs = 0; // prefix (n + 1 entries) and order (n entries) in `starts`
   };
   int n = 0;
@@ -76,7 +77,9 @@ struct cr_batch {
   Tables groups[kMaxGroups];          // views split into cost-balanced groups, one launch chain each
   int numGroups = 1;
   Tables subset;                      // views re-drawn after an overflow
-  hipStream_t side[kMaxGroups] = {};  // groups 1.. run on these (group 0 on the draw's stream)
+  // Groups 1.. run on these (group 0 on the draw's stream); in the graph of a
+  // single group, every second fine stage on side[1].
+  hipStream_t side[kMaxGroups] = {};
   hipEvent_t evFork = nullptr, evJoin[kMaxGroups] = {};
   int tilesPerGroup = 4;
   int banded = 0;                     // fine tile groups in XCD bands (1) or round-robin (0)
@@ -84,6 +87,7 @@ struct cr_batch {
   bool haveCounts = false;            // hostCounters hold every view's demand from a complete draw
   bool moved = false;                 // views' buffers changed since the tables were built
   bool laidOut = false, useGraph = true, graphValid = false, tuned = false;
+  bool drawn = false;                 // a draw of these views is behind: their capacities have held
   hipStream_t capStream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -248,6 +252,7 @@ cr_status buildTables(cr_batch* b, Tables& T, const std::vector<int>& idx) {
     if (list.empty()) continue;
     Tables::Stage S;
     S.variant = var;
+    for (int k : list) S.tiles += ps[k].numTiles;
     appendStage(st, S, longestFirst(tileCost, list), groups, most);
     if (S.blocks > 0) T.fine.push_back(S);
   }
@@ -298,23 +303,54 @@ cr_status buildAll(cr_batch* b) {
   return CR_OK;
 }
 
-cr_status launchTables(cr_batch* b, const Tables& T, hipStream_t stream) {
+// Whether a graph's fine stages of several pipe variants run in two chains side
+// by side: a variant's last tiles, one wave each over a list of hundreds of
+// entries, leave most of the chip idle, and small views are all last tiles.
+// 1x and 4x views: 3.6k tiles 188 -> 145 us a draw, 25k 408 -> 317, 60k 166 ->
+// 151, 183k 330 -> 319; with 540k, full of either variant, 767 -> 776.  The
+// branch itself costs some 8 us: with 169 tiles on one side 90 -> 98.
+bool forksFine(const Tables& T) {
+  int64_t chain[2] = {0, 0};
+  for (size_t i = 0; i < T.fine.size(); i++) chain[i & 1] += T.fine[i].tiles;
+  return std::min(chain[0], chain[1]) >= 512 && chain[0] + chain[1] <= 256 * 1024;
+}
+
+// One launch chain, or two for the fine stages.
+cr_status launchTables(cr_batch* b, const Tables& T, hipStream_t stream, bool twoFine = false) {
   const Params* pv = T.params.as<Params>();
   const int32_t* s = T.starts.as<int32_t>();
   launchSetupBatch(pv, s + T.setup.ofs, s + T.setup.orderOfs, T.setup.n, T.setup.blocks, stream);
   launchCoarseBatch(b->coarseThreads, pv, s + T.coarse.ofs, s + T.coarse.orderOfs, T.coarse.n, T.coarse.blocks,
                     stream);
-  for (const Tables::Stage& f : T.fine)
-    launchFineBatch(f.variant, b->tilesPerGroup, b->banded, pv, s + f.ofs, s + f.orderOfs, f.n, f.blocks, stream);
+  twoFine = twoFine && forksFine(T);
+  if (twoFine) {
+    CR_HIP(b->ctx, hipEventRecord(b->evFork, stream));
+    CR_HIP(b->ctx, hipStreamWaitEvent(b->side[1], b->evFork, 0));
+  }
+  for (size_t i = 0; i < T.fine.size(); i++) {
+    const Tables::Stage& f = T.fine[i];
+    launchFineBatch(f.variant, b->tilesPerGroup, b->banded, pv, s + f.ofs, s + f.orderOfs, f.n, f.blocks,
+                    twoFine && (i & 1) ? b->side[1] : stream);
+  }
+  if (twoFine) {
+    CR_HIP(b->ctx, hipEventRecord(b->evJoin[1], b->side[1]));
+    CR_HIP(b->ctx, hipStreamWaitEvent(stream, b->evJoin[1], 0));
+  }
   launchFinishBatch(pv, T.n, b->counters.as<Counters>(), b->hostCountersDev, stream);
   CR_HIP(b->ctx, hipGetLastError());
   return CR_OK;
 }
 
 // All groups: group 0 on `stream`, the others on side streams forked from
-// and joined back into it (parallel branches when captured in a graph).
+// and joined back into it (parallel branches when captured in a graph).  The
+// first draw runs them one after the other on `stream`, behind the uploads of
+// their tables.
 cr_status launchAllGroups(cr_batch* b, hipStream_t stream) {
-  if (b->numGroups <= 1) return launchTables(b, b->groups[0], stream);
+  if (b->numGroups <= 1 || !b->drawn) {
+    cr_status st = CR_OK;
+    for (int g = 0; g < b->numGroups && st == CR_OK; g++) st = launchTables(b, b->groups[g], stream);
+    return st;
+  }
   CR_HIP(b->ctx, hipEventRecord(b->evFork, stream));
   for (int g = 1; g < b->numGroups; g++) CR_HIP(b->ctx, hipStreamWaitEvent(b->side[g], b->evFork, 0));
   cr_status st = launchTables(b, b->groups[0], stream);
@@ -333,7 +369,8 @@ cr_status capture(cr_batch* b) {
   b->exec = nullptr;
   b->graph = nullptr;
   CR_HIP(ctx, hipStreamBeginCapture(b->capStream, hipStreamCaptureModeThreadLocal));
-  cr_status st = launchAllGroups(b, b->capStream);
+  cr_status st = b->numGroups <= 1 ? launchTables(b, b->groups[0], b->capStream, true)
+                                   : launchAllGroups(b, b->capStream);
   hipError_t e = hipStreamEndCapture(b->capStream, &b->graph);
   if (st != CR_OK) return st;
   CR_HIP(ctx, e);
@@ -423,6 +460,11 @@ cr_status drawBatch(cr_batch* b, hipStream_t stream, bool graph) {
   cr_status st = prepare(b);
   if (st != CR_OK) return st;
   b->retries = 0;
+  // The first draw is launched stage by stage: capturing costs more than the
+  // graph saves on it (8 small views, first draw: 585 us captured, 410 launched;
+  // later draws: 137 replayed, 143 launched), and queues that turn out too small
+  // void the graph.
+  graph = graph && b->drawn;
   if (graph && !b->graphValid) {
     st = capture(b);
     if (st != CR_OK) return st;
@@ -448,7 +490,9 @@ cr_status drawBatch(cr_batch* b, hipStream_t stream, bool graph) {
     last = std::max(last, s[kStampEnd]);
   }
   b->lastTicks = last > first ? last - first : 0;
-  return settleOverflow(b, stream);
+  st = settleOverflow(b, stream);
+  if (st == CR_OK) b->drawn = true;
+  return st;
 }
 
 // Device-to-device copies of the surfaces of views drawn without deferred

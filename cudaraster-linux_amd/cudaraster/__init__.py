@@ -543,7 +543,8 @@ def _stream_handle(stream):
 class Batch:
     """A batched multi-view draw (cr_batch_*): every view's surfaces, buffers
     and pipe are fixed at creation; draw() renders all of them, with one
-    launch per stage over all views, replayed from a captured hipGraph."""
+    launch per stage over all views, from the second draw on replayed from a
+    captured hipGraph."""
 
     def __init__(self, raster, views, keep=()):
         self._raster = raster
