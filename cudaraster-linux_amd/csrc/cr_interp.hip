@@ -79,15 +79,21 @@ __device__ __forceinline__ bool pixelTriangle(const InterpGeom& G, const InterpV
   return true;
 }
 
-// One lane per pixel, one grid row per image row, one grid layer per view.
+constexpr int kFwdTile = 16;
+
+// One lane per pixel, one 16x16-pixel tile per workgroup, one grid layer per
+// view.  Bound by the gathers of vertices: a tile's pixels share them in the
+// CU's cache, a row's hardly do.  16 views of 200k triangles, 512x512, 8
+// channels: 107 us in rows of 256 pixels, 82 in tiles (86 with every lane's
+// channels fetched ahead of its barycentrics).
 // vec4: C % 4 == 0 and attr / out 16-byte aligned, so channels move as
 // float4.
 template <int N>
-__global__ void __launch_bounds__(256) interpForwardKernel(const InterpGeom G, const InterpTable<N> T) {
+__global__ void __launch_bounds__(kFwdTile * kFwdTile) interpForwardKernel(const InterpGeom G, const InterpTable<N> T) {
   const InterpView& V = T.v[N == 1 ? 0 : blockIdx.z];
-  const int x = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  const int y = (int)blockIdx.y;
-  if (x >= G.width) return;
+  const int x = (int)(blockIdx.x * kFwdTile + threadIdx.x % kFwdTile);
+  const int y = (int)(blockIdx.y * kFwdTile + threadIdx.x / kFwdTile);
+  if (x >= G.width || y >= G.height) return;
   const int64_t p = (int64_t)y * G.width + x;
   const int C = G.numChannels;
   const bool vec4 = V.vec4 != 0;
@@ -581,8 +587,9 @@ __global__ void __launch_bounds__(256) fixedToFloatKernel(const InterpTable<N> T
 
 template <int N>
 static void forwardViews(const InterpGeom& G, const InterpTable<N>& T, int n, hipStream_t stream) {
-  hipLaunchKernelGGL((interpForwardKernel<N>), dim3((unsigned)((G.width + 255) / 256), (unsigned)G.height, (unsigned)n),
-                     dim3(256), 0, stream, G, T);
+  hipLaunchKernelGGL((interpForwardKernel<N>), dim3((unsigned)((G.width + kFwdTile - 1) / kFwdTile),
+                     (unsigned)((G.height + kFwdTile - 1) / kFwdTile), (unsigned)n), dim3(kFwdTile * kFwdTile), 0,
+                     stream, G, T);
 }
 
 template <int N>
