@@ -8,7 +8,7 @@ call returns when the frame is complete and the overflow counters have been
 read back).  Inputs are resident in HBM before timing starts; the draws
 are timed by a native loop over the C ABI.  Prints one
 JSON line: Mtris/s as `value`, Gfragments/s beside it, the roofline of the
-dominant kernel (timed with HIP events on the draw stream) and the CPU
+dominant kernel (timed with the library's device clock stamps) and the CPU
 oracle's throughput on the same workload as `cpu_baseline`.
 """
 from __future__ import annotations
@@ -52,21 +52,21 @@ def setup_algorithmic_bytes(scene, c, visible_subtris):
     """Setup + binning: indices (12 B) and three clip positions (16 B each)
     read per triangle; per visible subtriangle a 16 B header, a 64 B data
     record and its 4 B source index written; 16 B per bin-queue entry (slot
-    and snapped vertices) and 8 B per (bin, chunk) count/offset pair written."""
+    and snapped vertices) and 4 B per (bin, chunk) of queue addresses written."""
     chunks = (scene.num_tris + 1023) // 1024
     bins = ((scene.width + 127) // 128) * ((scene.height + 127) // 128)
     return (scene.num_tris * (12 + 3 * 16) + visible_subtris * (16 + 64 + 4)
-            + c["bin_entries"] * 16 + bins * chunks * 8)
+            + c["bin_entries"] * 16 + bins * chunks * 4)
 
 
 def coarse_algorithmic_bytes(scene, c, visible_subtris):
     """Coarse: every 16 B bin-queue entry and the per-(bin, chunk)
-    counts/offsets read, every tile-list entry (4 B) and per-tile start/count
+    queue addresses read, every tile-list entry (4 B) and per-tile start/count
     (8 B) written."""
     chunks = (scene.num_tris + 1023) // 1024
     bins = ((scene.width + 127) // 128) * ((scene.height + 127) // 128)
     tiles = ((scene.width + 7) // 8) * ((scene.height + 7) // 8)
-    return c["bin_entries"] * 16 + bins * chunks * 8 + c["tile_list_entries"] * 4 + tiles * 8
+    return c["bin_entries"] * 16 + bins * chunks * 4 + c["tile_list_entries"] * 4 + tiles * 8
 
 
 def measured_traffic(kernel, workload_key, triid):
@@ -166,8 +166,8 @@ def multi_view_ratio(reps=5, triid=True):
             cr.drawTriangles()
 
     plain_pass()
-    # GPU time of the plain draws: per view, the stage events of its draw
-    # (reset, setup+bin, coarse, fine) summed over the 64 views.
+    # GPU time of the plain draws: per view, the stage times of its draw
+    # (setup+bin, coarse, fine) summed over the 64 views.
     plain_gpu_ms = 0.0
     for k, sc in enumerate(views):
         col, dep, tid = plain_surf[k]
@@ -459,7 +459,7 @@ def plain_workload_leg(name, steps=10, warmup=2, triid=True, cpu=True):
         kernels[kname]["frac"] = kernels[kname]["GBps"] / HBM_PEAK_GBS if kernels[kname]["GBps"] else None
     ms = elapsed / steps * 1e3
     out = {"workload": desc, "triangles": scene.num_tris, "steps": steps, "ms_per_step": ms,
-           "timing": "native C loop over the C ABI; stage_ms from the library's stage events",
+           "timing": "native C loop over the C ABI; stage_ms from the library's stage stamps",
            "ms_per_step_python": elapsed_py / steps * 1e3,
            "gpu_ms_per_draw": statistics.median(gpu_draw) * 1e3,
            "mtris_per_s_gpu_time": scene.num_tris / statistics.median(gpu_draw) / 1e6,
@@ -558,7 +558,7 @@ def main():
 
     avg = {k: v / args.steps for k, v in stage.items()}
     # Per-kernel roofline: algorithmic bytes of one launch over its average
-    # duration (HIP events recorded around each kernel on the draw stream).
+    # duration (the library's device clock stamps: stage start to stage start).
     kernels = {}
     for key, kname, fn in (("setupTime", "setupBinKernel", lambda: setup_algorithmic_bytes(scene, counters, visible)),
                            ("coarseTime", "coarseKernel", lambda: coarse_algorithmic_bytes(scene, counters, visible)),
@@ -583,9 +583,9 @@ def main():
         "warmup": args.warmup,
         "ms_per_step": ms,
         "timing": "native C loop over the C ABI (cudaraster-linux_amd/bench_native/plain_draws.cpp); "
-                  "stage_ms from the library's stage events",
+                  "stage_ms from the library's stage stamps",
         "ms_per_step_python": elapsed_py / args.steps * 1e3,
-        # The draw's GPU time from the first stage to the last (HIP events,
+        # The draw's GPU time from the first stage to the last (clock stamps,
         # median over the steps) and the triangle rate over it.
         "gpu_ms_per_draw": statistics.median(gpu_draw) * 1e3,
         "mtris_per_s_gpu_time": scene.num_tris / statistics.median(gpu_draw) / 1e6,

@@ -136,7 +136,7 @@ typedef struct cr_pipe_desc {
 } cr_pipe_desc;
 
 /* CudaRaster::Stats (CudaRaster.hpp:45-51): seconds per stage of the last
- * draw, from HIP events.  Triangle setup and binning run as one kernel:
+ * draw, from device clock stamps.  Triangle setup and binning run as one kernel:
  * setup_time covers both and bin_time is 0. */
 typedef struct cr_stats {
     float setup_time;
@@ -321,7 +321,8 @@ cr_status cr_set_debug_params(cr_context* ctx, const cr_debug_params* p);
  * The reference draws one view per drawTriangles() call, each synchronous.
  * A batch draws many independent views -- each with its own surfaces,
  * buffers, pipe, resolution and sample count -- with one launch per stage
- * over all views, replayed from a captured hipGraph.  Every view's output is
+ * over all views, from the second draw on replayed from a captured hipGraph.
+ * Every view's output is
  * bit-identical to a plain draw of the same state (cr_set_surfaces,
  * cr_set_pixel_pipe, cr_set_*_buffer, cr_deferred_clear, cr_draw_triangles).
  *
@@ -352,7 +353,7 @@ typedef struct cr_batch_info {
     int32_t tuned;                 /* 1: cr_batch_autotune has run */
     int64_t retries;               /* capacity grow rounds of the last draw */
     int64_t reserved_bytes;        /* device bytes of the batch's intermediate buffers */
-    float last_gpu_ms;             /* GPU time of the last draw's launch (events around it) */
+    float last_gpu_ms;             /* GPU time of the last draw's launch (first stage's start to last end) */
     float tuned_gpu_ms;            /* best GPU time seen by the autotuner */
     int32_t fine_banded;           /* 1: fine tile groups in per-XCD bands; 0: dealt round-robin */
     int32_t coarse_threads;        /* coarse-stage workgroup size in use */
