@@ -15,9 +15,10 @@
 //    entry j against the tile's hierarchical Z; the survivors, gathered over
 //    chunks into batches of up to 32, are set up one per lane (tile-relative
 //    edge thresholds per sample, depth plane per sample) into an LDS record
-//    array, and the wave then walks the records with broadcast LDS reads --
-//    per (triangle, tile) the lanes only do integer compares, one depth add
-//    per sample and register selects;
+//    array, which the wave then walks -- record by record with broadcast reads
+//    where fragments are blended in order, else every lane the records that
+//    its pixel's mask names.  Per record the lanes only do integer compares,
+//    one depth add per sample and register selects;
 //  * for Replace and DepthOnly blending the colour written to a sample is
 //    the shaded colour of the last fragment that passed there, so shading is
 //    deferred: the loop records (subtriangle slot, centroid) per sample and
