@@ -9,7 +9,8 @@
 // subtriangles take consecutive slots from a device counter (slots beyond
 // numTris), their source index goes to subtriTri, and misc holds the base.
 //
-// The clip polygon lives in registers, one vertex per lane of the wave,
+// The clip polygon lives in registers, one vertex per lane of the wave, or,
+// where several of a wave's triangles are clipped, in scratch memory per lane,
 // instead of the reference's per-thread shared-memory array.
 #include "cr_device.h"
 
@@ -196,15 +197,18 @@ __device__ __forceinline__ void setupTriangle(const PP& P, Header* th, TriData* 
       (zmin & 0xFFFFF000u) | (f01 << 6) | (f12 << 2) | (f20 >> 2));
 }
 
-// ---- clipping: one triangle by the whole wave ---------------------------------
+// ---- clipping -------------------------------------------------------------------
 //
-// Lane i holds vertex i of the clip polygon (at most 9) as its barycentrics;
-// vertices past the polygon's end take no part.  Few triangles are clipped,
-// so a wave clips them one after another: with a polygon per lane, in arrays
-// indexed at run time, a single clipped triangle held its 1024-triangle
-// workgroup up for 400k cycles of dependent scratch accesses (4M small
-// triangles among 1024 clipped ones, setup 382 -> 237 us with this and the
-// wide boxes below).
+// A wave's only clipped triangle is clipped by the whole wave: lane i holds
+// vertex i of the clip polygon (at most 9) as its barycentrics; vertices past
+// the polygon's end take no part.  With more of them, every lane clips its own,
+// in an array indexed at run time, and the wave takes all slots with one
+// addition to the draw's counter.  One after another they would take as many
+// times as long as there are: setup of 1024 triangles with 2 / 64 clipped of
+// every 64 50 / 560 us, by lanes 50 / 55; of 100k, then bound by an addition per
+// triangle, 73 / 1208 and 63 / 70.  A single one takes the 1024 triangles 30 us
+// by the wave, 48 by its lane; 1M small triangles with 256 large clipped ones
+// among them 66 and 98.
 struct ClipVert { float b0, b1; };
 
 // Vertex of lane `from`.
@@ -269,75 +273,162 @@ __device__ __forceinline__ float4 lerpClip(const float4& o, const float4& d1, co
                      fmaf(d2.z, b.b1, fmaf(d1.z, b.b0, o.z)), fmaf(d2.w, b.b1, fmaf(d1.w, b.b0, o.w)));
 }
 
-__device__ __forceinline__ float4 laneValue(const float4& v, int j) {
-  return make_float4(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v.x), j)),
-                     __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v.y), j)),
-                     __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v.z), j)),
-                     __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v.w), j)));
-}
-
 struct ClipResult { int numSub, base; };
 
-// Slow path, kept out of line, called by whole waves: frustum clip and fan
-// (TriangleSetup.inl:326-412) of the triangles of the lanes in `todo`, one
-// after another; lane f sets up fan triangle f.  Returns, per lane in todo,
-// the number of subtriangles written (0 when the slot allocation overflowed)
-// and their first slot.
-__device__ __noinline__ ClipResult setupClipped(const ClipCtx P, uint64_t todo, int tOwn) {
-  const int lane = (int)(threadIdx.x & 63);
-  ClipResult out = {0, tOwn};
-  int3 vidxOwn = make_int3(0, 0, 0);
-  float4 own0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), own1 = own0, own2 = own0;
-  if ((todo >> lane) & 1u) {
-    const int32_t* ip = P.indices + (int64_t)tOwn * 3;
-    vidxOwn = make_int3(ip[0], ip[1], ip[2]);
-    own0 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidxOwn.x * P.vertexStride);
-    own1 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidxOwn.y * P.vertexStride);
-    own2 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidxOwn.z * P.vertexStride);
+// clipPolygon by one lane, its polygon in an array.
+__device__ __forceinline__ int clipPolygonLane(float* out, const float* in, int numIn, float v0, float v1, float v2) {
+  int numOut = 0;
+  if (numIn >= 3) {
+    int ai = (numIn - 1) * 2;
+    float av = fmaf(v2, in[ai + 1], fmaf(v1, in[ai + 0], v0));
+    for (int bi = 0; bi < numIn * 2; bi += 2) {
+      const float bv = fmaf(v2, in[bi + 1], fmaf(v1, in[bi + 0], v0));
+      if (av * bv < 0.0f && numOut < 18) {             // (at most 9 vertices)
+        const float bc = av / (av - bv);
+        const float ac = 1.0f - bc;
+        out[numOut + 0] = fmaf(in[ai + 0], ac, in[bi + 0] * bc);
+        out[numOut + 1] = fmaf(in[ai + 1], ac, in[bi + 1] * bc);
+        numOut += 2;
+      }
+      if (bv >= 0.0f && numOut < 18) {
+        out[numOut + 0] = in[bi + 0];
+        out[numOut + 1] = in[bi + 1];
+        numOut += 2;
+      }
+      ai = bi;
+      av = bv;
+    }
   }
-  for (; todo != 0; todo &= todo - 1) {
-    const int j = (int)__builtin_ctzll(todo);
-    const int t = __builtin_amdgcn_readlane(tOwn, j);
-    const int3 vidx = make_int3(__builtin_amdgcn_readlane(vidxOwn.x, j), __builtin_amdgcn_readlane(vidxOwn.y, j),
-                                __builtin_amdgcn_readlane(vidxOwn.z, j));
-    const float4 ov0 = laneValue(own0, j), ov1 = laneValue(own1, j), ov2 = laneValue(own2, j);
-    const float4 od1 = make_float4(ov1.x - ov0.x, ov1.y - ov0.y, ov1.z - ov0.z, ov1.w - ov0.w);
-    const float4 od2 = make_float4(ov2.x - ov0.x, ov2.y - ov0.y, ov2.z - ov0.z, ov2.w - ov0.w);
-    ClipVert v;
-    const int numVerts = clipTriangle(v, ov0, ov1, ov2, od1, od2);
-    const ClipVert c0 = vertOf(v, 0), c1 = vertOf(v, (lane + 1) & 63), c2 = vertOf(v, (lane + 2) & 63);
-    const float4 v0 = lerpClip(ov0, od1, od2, c0), v1 = lerpClip(ov0, od1, od2, c1), v2 = lerpClip(ov0, od1, od2, c2);
-    I2 p0, p1, p2, lo, hi, d1, d2;
-    float rcpW[3];
-    int32_t area;
+  return numOut >> 1;
+}
+
+// The clip of the triangles of the lanes in `todo`, each by its own lane.
+__device__ __forceinline__ ClipResult setupClippedLanes(const ClipCtx& P, uint64_t todo, int t) {
+  const int lane = (int)(threadIdx.x & 63);
+  const bool mine = ((todo >> lane) & 1u) != 0;
+  float bary[18];
+  int numVerts = 0, numSub = 0;
+  int3 vidx = make_int3(0, 0, 0);
+  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f), od1 = o, od2 = o;
+  auto vertex = [&](int i) { return lerpClip(o, od1, od2, {bary[2 * i], bary[2 * i + 1]}); };
+  I2 p0, p1, p2, lo, hi, d1, d2;
+  float rcpW[3];
+  int32_t area;
+  if (mine) {
+    const int32_t* ip = P.indices + (int64_t)t * 3;
+    vidx = make_int3(ip[0], ip[1], ip[2]);
+    o = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.x * P.vertexStride);
+    const float4 b = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.y * P.vertexStride);
+    const float4 c = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.z * P.vertexStride);
+    od1 = make_float4(b.x - o.x, b.y - o.y, b.z - o.z, b.w - o.w);
+    od2 = make_float4(c.x - o.x, c.y - o.y, c.z - o.z, c.w - o.w);
+    float temp[18];
+    bary[0] = 0.0f; bary[1] = 0.0f;
+    bary[2] = 1.0f; bary[3] = 0.0f;
+    bary[4] = 0.0f; bary[5] = 1.0f;
+    numVerts = 3;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      if ((o.w < fabsf(comp(o, a))) | (b.w < fabsf(comp(b, a))) | (c.w < fabsf(comp(c, a)))) {
+        numVerts = clipPolygonLane(temp, bary, numVerts, o.w + comp(o, a), od1.w + comp(od1, a), od2.w + comp(od2, a));
+        numVerts = clipPolygonLane(bary, temp, numVerts, o.w - comp(o, a), od1.w - comp(od1, a), od2.w - comp(od2, a));
+      }
+    }
+    const float4 v0 = vertex(0);
+    float4 v1 = vertex(1);
+    for (int i = 2; i < numVerts; i++) {
+      const float4 v2 = vertex(i);
+      snap(P, v0, v1, v2, p0, p1, p2, rcpW, lo, hi);
+      if (prepare(P, p0, p1, p2, lo, hi, d1, d2, area) == 0) numSub++;
+      v1 = v2;
+    }
+  }
+  // One addition to the slot counter for the wave.
+  const uint32_t need = numSub > 1 ? (uint32_t)numSub : 0u;
+  const uint32_t scan = waveScan(need);
+  const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)scan, 63);
+  uint32_t at = 0;
+  if (lane == 0 && all) at = atomicAdd(&P.counters->numSubtris, all);
+  at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+  ClipResult out = {0, t};
+  if (!mine) return out;
+  if (numSub > 1) out.base = P.numTris + (int)(at + scan - need);
+  const bool over = numSub > 1 && out.base + numSub > P.maxSubtris;
+  P.triSubtris[t] = (uint8_t)numSub;
+  if (numSub > 1) P.triHeader[t].misc = (uint32_t)out.base;
+  if (over) {
+    atomicOr(&P.counters->overflow, 1u);
+    return out;
+  }
+  out.numSub = numSub;
+  int slot = out.base;
+  const float4 v0 = vertex(0);
+  float4 v1 = vertex(1);
+  for (int i = 2; i < numVerts; i++) {
+    const float4 v2 = vertex(i);
     snap(P, v0, v1, v2, p0, p1, p2, rcpW, lo, hi);
-    const bool vis = lane + 2 < numVerts && prepare(P, p0, p1, p2, lo, hi, d1, d2, area) == 0;
-    const uint64_t vm = __ballot(vis);
-    int numSub = (int)__popcll(vm);
-    int base = t;
-    if (numSub > 1) {
-      int at = 0;
-      if (lane == 0) at = P.numTris + (int)atomicAdd(&P.counters->numSubtris, (uint32_t)numSub);
-      base = __builtin_amdgcn_readfirstlane(at);
-    }
-    const bool over = numSub > 1 && base + numSub > P.maxSubtris;
-    if (lane == 0) {
-      P.triSubtris[t] = (uint8_t)numSub;
-      if (numSub > 1) P.triHeader[t].misc = (uint32_t)base;
-      if (over) atomicOr(&P.counters->overflow, 1u);
-    }
-    if (vis && !over) {
-      const int slot = base + (int)__popcll(vm & ((1ull << lane) - 1ull));
-      setupTriangle(P, &P.triHeader[slot], &P.triData[slot], vidx, v0, v1, v2, make_float2(c0.b0, c0.b1),
-                    make_float2(c1.b0, c1.b1), make_float2(c2.b0, c2.b1), p0, p1, p2, rcpW, d1, d2, area);
+    if (prepare(P, p0, p1, p2, lo, hi, d1, d2, area) == 0) {
+      setupTriangle(P, &P.triHeader[slot], &P.triData[slot], vidx, v0, v1, v2, make_float2(bary[0], bary[1]),
+                    make_float2(bary[2 * i - 2], bary[2 * i - 1]), make_float2(bary[2 * i], bary[2 * i + 1]), p0, p1,
+                    p2, rcpW, d1, d2, area);
       if (slot >= P.numTris) P.subtriTri[slot - P.numTris] = (uint32_t)t;
+      slot++;
     }
-    if (lane == j) {
-      out.numSub = over ? 0 : numSub;
-      out.base = base;
-    }
+    v1 = v2;
   }
   return out;
+}
+
+// The clip of triangle t (uniform) by the whole wave; lane f sets up fan
+// triangle f.
+__device__ __forceinline__ ClipResult setupClippedWave(const ClipCtx& P, int t) {
+  const int lane = (int)(threadIdx.x & 63);
+  const int32_t* ip = P.indices + (int64_t)t * 3;
+  const int3 vidx = make_int3(ip[0], ip[1], ip[2]);
+  const float4 ov0 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.x * P.vertexStride);
+  const float4 ov1 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.y * P.vertexStride);
+  const float4 ov2 = *reinterpret_cast<const float4*>(P.vertices + (int64_t)vidx.z * P.vertexStride);
+  const float4 od1 = make_float4(ov1.x - ov0.x, ov1.y - ov0.y, ov1.z - ov0.z, ov1.w - ov0.w);
+  const float4 od2 = make_float4(ov2.x - ov0.x, ov2.y - ov0.y, ov2.z - ov0.z, ov2.w - ov0.w);
+  ClipVert v;
+  const int numVerts = clipTriangle(v, ov0, ov1, ov2, od1, od2);
+  const ClipVert c0 = vertOf(v, 0), c1 = vertOf(v, (lane + 1) & 63), c2 = vertOf(v, (lane + 2) & 63);
+  const float4 v0 = lerpClip(ov0, od1, od2, c0), v1 = lerpClip(ov0, od1, od2, c1), v2 = lerpClip(ov0, od1, od2, c2);
+  I2 p0, p1, p2, lo, hi, d1, d2;
+  float rcpW[3];
+  int32_t area;
+  snap(P, v0, v1, v2, p0, p1, p2, rcpW, lo, hi);
+  const bool vis = lane + 2 < numVerts && prepare(P, p0, p1, p2, lo, hi, d1, d2, area) == 0;
+  const uint64_t vm = __ballot(vis);
+  const int numSub = (int)__popcll(vm);
+  int base = t;
+  if (numSub > 1) {
+    int at = 0;
+    if (lane == 0) at = P.numTris + (int)atomicAdd(&P.counters->numSubtris, (uint32_t)numSub);
+    base = __builtin_amdgcn_readfirstlane(at);
+  }
+  const bool over = numSub > 1 && base + numSub > P.maxSubtris;
+  if (lane == 0) {
+    P.triSubtris[t] = (uint8_t)numSub;
+    if (numSub > 1) P.triHeader[t].misc = (uint32_t)base;
+    if (over) atomicOr(&P.counters->overflow, 1u);
+  }
+  if (vis && !over) {
+    const int slot = base + (int)__popcll(vm & ((1ull << lane) - 1ull));
+    setupTriangle(P, &P.triHeader[slot], &P.triData[slot], vidx, v0, v1, v2, make_float2(c0.b0, c0.b1),
+                  make_float2(c1.b0, c1.b1), make_float2(c2.b0, c2.b1), p0, p1, p2, rcpW, d1, d2, area);
+    if (slot >= P.numTris) P.subtriTri[slot - P.numTris] = (uint32_t)t;
+  }
+  return {over ? 0 : numSub, base};
+}
+
+// Slow path, kept out of line, called by whole waves: frustum clip and fan
+// (TriangleSetup.inl:326-412) of the triangles of the lanes in `todo` (not
+// empty).  Returns, per lane in todo, the number of subtriangles written (0
+// when the slot allocation overflowed) and their first slot.
+__device__ __noinline__ ClipResult setupClipped(const ClipCtx P, uint64_t todo, int t) {
+  if (__popcll(todo) > 1) return setupClippedLanes(P, todo, t);
+  return setupClippedWave(P, __builtin_amdgcn_readlane(t, (int)__builtin_ctzll(todo)));
 }
 
 // Outcome of one triangle's setup, as the reference's setup counters
