@@ -73,7 +73,7 @@ struct cr_batch {
   DevBuf tileStart, tileCount, tileList, tileSegNext, counters, saved;
   Counters* hostCounters = nullptr;   // pinned, one block per view, written by the draws' finish kernels
   Counters* hostCountersDev = nullptr;   // their device address
-  bool countersClean = false;         // every view's last draw was queued whole: it leaves its counters cleared
+  bool countersClean = false;         // every view's last draw has ended: it left its counters cleared
   Tables groups[kMaxGroups];          // views split into cost-balanced groups, one launch chain each
   int numGroups = 1;
   Tables subset;                      // views re-drawn after an overflow
@@ -414,7 +414,6 @@ cr_status patchBuffers(cr_batch* b, hipStream_t stream) {
     }
   }
   CR_HIP(b->ctx, hipGetLastError());
-  b->moved = false;
   return CR_OK;
 }
 
@@ -449,15 +448,27 @@ cr_status settleOverflow(cr_batch* b, hipStream_t stream) {
     b->countersClean = false;
     st = launchTables(b, b->subset, stream);
     if (st != CR_OK) return st;
-    b->countersClean = true;
     CR_HIP(b->ctx, hipStreamSynchronize(stream));
+    b->countersClean = true;
   }
+}
+
+// A batch draw waits for its counters: refused, before anything of the batch
+// changes, on a stream that captures (its launches would be recorded instead of
+// run, the counters neither cleared nor the moved buffers written).
+cr_status refuseCapture(cr_batch* b, hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  CR_HIP(b->ctx, hipStreamIsCapturing(stream, &cap));
+  if (cap != hipStreamCaptureStatusNone)
+    return fail(b->ctx, CR_ERR_DEVICE, "batch: the draw waits for its counters, which a capturing stream cannot");
+  return CR_OK;
 }
 
 cr_status drawBatch(cr_batch* b, hipStream_t stream, bool graph) {
   cr_context* ctx = b->ctx;
   CR_HIP(ctx, hipSetDevice(ctx->device));
-  cr_status st = prepare(b);
+  cr_status st = refuseCapture(b, stream);
+  if (st == CR_OK) st = prepare(b);
   if (st != CR_OK) return st;
   b->retries = 0;
   // The first draw is launched stage by stage: capturing costs more than the
@@ -479,8 +490,9 @@ cr_status drawBatch(cr_batch* b, hipStream_t stream, bool graph) {
     st = launchAllGroups(b, stream);
     if (st != CR_OK) return st;
   }
-  b->countersClean = true;
   CR_HIP(ctx, hipStreamSynchronize(stream));
+  b->countersClean = true;
+  b->moved = false;
   // GPU time: the first stage's start to the last view's end.
   uint64_t first = UINT64_MAX, last = 0;
   for (size_t i = 0; i < b->views.size(); i++) {
@@ -629,7 +641,8 @@ cr_status cr_batch_autotune(cr_batch* b, void* stream_) {
   cr_context* ctx = b->ctx;
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   CR_HIP(ctx, hipSetDevice(ctx->device));
-  cr_status st = prepare(b);
+  cr_status st = refuseCapture(b, stream);
+  if (st == CR_OK) st = prepare(b);
   if (st == CR_OK) st = saveSurfaces(b, stream, false);
   // 1. Exact per-view queue demand (the draw grows whatever overflows).
   if (st == CR_OK) st = drawBatch(b, stream, false);
