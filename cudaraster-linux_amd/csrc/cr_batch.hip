@@ -661,6 +661,8 @@ cr_status cr_batch_autotune(cr_batch* b, void* stream_) {
   // 3. Fine-stage workgroup shape and placement: the fastest combination of
   //    the compiled shapes and banded / round-robin tile groups (the stages
   //    list views longest-first by the measured entries per bin and tile).
+  //    What is timed is what later draws run: the captured graph with its
+  //    parallel branches (rep 0 captures it), unless graphs are off.
   int bestW = b->tilesPerGroup, bestBanded = b->banded, bestCoarse = b->coarseThreads;
   float bestMs = 1e30f;
   const double tick = clockTick(b->device) * 1e3;
@@ -677,7 +679,7 @@ cr_status cr_batch_autotune(cr_batch* b, void* stream_) {
       float ms[3];
       for (int rep = 0; rep < 4; rep++) {
         st = saveSurfaces(b, stream, true);
-        if (st == CR_OK) st = drawBatch(b, stream, false);
+        if (st == CR_OK) st = drawBatch(b, stream, b->useGraph);
         if (st != CR_OK) return st;
         if (rep > 0) ms[rep - 1] = (float)((double)b->lastTicks * tick);
       }
@@ -705,7 +707,7 @@ cr_status cr_batch_autotune(cr_batch* b, void* stream_) {
     float ms[3];
     for (int rep = 0; rep < 4; rep++) {
       st = saveSurfaces(b, stream, true);
-      if (st == CR_OK) st = drawBatch(b, stream, false);
+      if (st == CR_OK) st = drawBatch(b, stream, b->useGraph);
       if (st != CR_OK) return st;
       if (rep > 0) ms[rep - 1] = (float)((double)b->lastTicks * tick);
     }
