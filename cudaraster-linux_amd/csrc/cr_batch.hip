@@ -77,10 +77,11 @@ struct cr_batch {
   Tables groups[kMaxGroups];          // views split into cost-balanced groups, one launch chain each
   int numGroups = 1;
   Tables subset;                      // views re-drawn after an overflow
-  // Groups 1.. run on these (group 0 on the draw's stream); in the graph of a
-  // single group, every second fine stage on side[1].
-  hipStream_t side[kMaxGroups] = {};
-  hipEvent_t evFork = nullptr, evJoin[kMaxGroups] = {};
+  // Streams and events of the graph's parallel branches, used in captures only:
+  // groups 1.. (group 0 on the capturing stream), and every second fine stage
+  // of a single group.
+  hipStream_t side[kMaxGroups] = {}, fineSide = nullptr;
+  hipEvent_t evFork = nullptr, evJoin[kMaxGroups] = {}, evFineFork = nullptr, evFineJoin = nullptr;
   int tilesPerGroup = 4;
   int banded = 0;                     // fine tile groups in XCD bands (1) or round-robin (0)
   int coarseThreads = 256;            // coarse workgroup size
@@ -259,8 +260,16 @@ cr_status buildTables(cr_batch* b, Tables& T, const std::vector<int>& idx) {
   if (most >= (int64_t)1 << 30) return fail(ctx, CR_ERR_OVERFLOW, "batch: more than 2^30 workgroups in one stage");
   CR_HIP(ctx, T.params.ensure((size_t)std::max(n, 1) * sizeof(Params)));
   CR_HIP(ctx, T.starts.ensure(st.size() * sizeof(int32_t)));
-  if (n > 0) CR_HIP(ctx, hipMemcpy(T.params.ptr, ps.data(), (size_t)n * sizeof(Params), hipMemcpyHostToDevice));
-  CR_HIP(ctx, hipMemcpy(T.starts.ptr, st.data(), st.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+  // On a stream of the batch's own, and waited for: whatever stream a draw or
+  // its graph's branches run on, the tables are there.
+  hipError_t e = hipSuccess;
+  if (n > 0)
+    e = hipMemcpyAsync(T.params.ptr, ps.data(), (size_t)n * sizeof(Params), hipMemcpyHostToDevice, b->capStream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(T.starts.ptr, st.data(), st.size() * sizeof(int32_t), hipMemcpyHostToDevice, b->capStream);
+  const hipError_t waited = hipStreamSynchronize(b->capStream);
+  CR_HIP(ctx, e);
+  CR_HIP(ctx, waited);
   T.n = n;
   T.members = idx;
   return CR_OK;
@@ -324,33 +333,36 @@ cr_status launchTables(cr_batch* b, const Tables& T, hipStream_t stream, bool tw
                     stream);
   twoFine = twoFine && forksFine(T);
   if (twoFine) {
-    CR_HIP(b->ctx, hipEventRecord(b->evFork, stream));
-    CR_HIP(b->ctx, hipStreamWaitEvent(b->side[1], b->evFork, 0));
+    CR_HIP(b->ctx, hipEventRecord(b->evFineFork, stream));
+    CR_HIP(b->ctx, hipStreamWaitEvent(b->fineSide, b->evFineFork, 0));
   }
   for (size_t i = 0; i < T.fine.size(); i++) {
     const Tables::Stage& f = T.fine[i];
     launchFineBatch(f.variant, b->tilesPerGroup, b->banded, pv, s + f.ofs, s + f.orderOfs, f.n, f.blocks,
-                    twoFine && (i & 1) ? b->side[1] : stream);
+                    twoFine && (i & 1) ? b->fineSide : stream);
   }
   if (twoFine) {
-    CR_HIP(b->ctx, hipEventRecord(b->evJoin[1], b->side[1]));
-    CR_HIP(b->ctx, hipStreamWaitEvent(stream, b->evJoin[1], 0));
+    CR_HIP(b->ctx, hipEventRecord(b->evFineJoin, b->fineSide));
+    CR_HIP(b->ctx, hipStreamWaitEvent(stream, b->evFineJoin, 0));
   }
   launchFinishBatch(pv, T.n, b->counters.as<Counters>(), b->hostCountersDev, stream);
   CR_HIP(b->ctx, hipGetLastError());
   return CR_OK;
 }
 
-// All groups: group 0 on `stream`, the others on side streams forked from
-// and joined back into it (parallel branches when captured in a graph).  The
-// first draw runs them one after the other on `stream`, behind the uploads of
-// their tables.
+// All groups launched one after the other on `stream`.  (Only a graph runs them
+// side by side: direct launches of freshly built groups on forked streams have
+// faulted the GPU for a cause that was not found.)
 cr_status launchAllGroups(cr_batch* b, hipStream_t stream) {
-  if (b->numGroups <= 1 || !b->drawn) {
-    cr_status st = CR_OK;
-    for (int g = 0; g < b->numGroups && st == CR_OK; g++) st = launchTables(b, b->groups[g], stream);
-    return st;
-  }
+  cr_status st = CR_OK;
+  for (int g = 0; g < b->numGroups && st == CR_OK; g++) st = launchTables(b, b->groups[g], stream);
+  return st;
+}
+
+// All groups as parallel branches of the graph that capStream captures.
+cr_status captureGroups(cr_batch* b) {
+  hipStream_t stream = b->capStream;
+  if (b->numGroups <= 1) return launchTables(b, b->groups[0], stream, true);
   CR_HIP(b->ctx, hipEventRecord(b->evFork, stream));
   for (int g = 1; g < b->numGroups; g++) CR_HIP(b->ctx, hipStreamWaitEvent(b->side[g], b->evFork, 0));
   cr_status st = launchTables(b, b->groups[0], stream);
@@ -369,8 +381,7 @@ cr_status capture(cr_batch* b) {
   b->exec = nullptr;
   b->graph = nullptr;
   CR_HIP(ctx, hipStreamBeginCapture(b->capStream, hipStreamCaptureModeThreadLocal));
-  cr_status st = b->numGroups <= 1 ? launchTables(b, b->groups[0], b->capStream, true)
-                                   : launchAllGroups(b, b->capStream);
+  cr_status st = captureGroups(b);
   hipError_t e = hipStreamEndCapture(b->capStream, &b->graph);
   if (st != CR_OK) return st;
   CR_HIP(ctx, e);
@@ -590,6 +601,9 @@ cr_status cr_batch_create(cr_context* ctx, const cr_view* views, int32_t numView
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->capStream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&b->hostCountersDev, b->hostCounters, 0);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&b->evFork, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&b->evFineFork, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&b->evFineJoin, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->fineSide, hipStreamNonBlocking);
   for (int g = 1; g < kMaxGroups && e == hipSuccess; g++) {
     e = hipStreamCreateWithFlags(&b->side[g], hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->evJoin[g], hipEventDisableTiming);
@@ -624,7 +638,9 @@ cr_status cr_batch_destroy(cr_batch* b) {
     if (b->side[g]) (void)hipStreamDestroy(b->side[g]);
     if (b->evJoin[g]) (void)hipEventDestroy(b->evJoin[g]);
   }
-  if (b->evFork) (void)hipEventDestroy(b->evFork);
+  if (b->fineSide) (void)hipStreamDestroy(b->fineSide);
+  for (hipEvent_t e : {b->evFork, b->evFineFork, b->evFineJoin})
+    if (e) (void)hipEventDestroy(e);
   delete b;
   return CR_OK;
 }
@@ -697,10 +713,10 @@ cr_status cr_batch_autotune(cr_batch* b, void* stream_) {
   b->banded = bestBanded;
   b->coarseThreads = bestCoarse;
   // 4. Concurrent view groups: the views split into K cost-balanced groups
-  //    whose launch chains run side by side (K = 1, 2 or 4).
+  //    whose launch chains run side by side (K = 1, 2 or 4) in the graph.
   int bestK = 1;
   for (int K : {2, 4}) {
-    if (K > (int)b->views.size()) break;
+    if (K > (int)b->views.size() || !b->useGraph) break;
     b->numGroups = K;
     st = buildAll(b);
     if (st != CR_OK) return st;

@@ -357,7 +357,7 @@ typedef struct cr_batch_info {
     float tuned_gpu_ms;            /* best GPU time seen by the autotuner */
     int32_t fine_banded;           /* 1: fine tile groups in per-XCD bands; 0: dealt round-robin */
     int32_t coarse_threads;        /* coarse-stage workgroup size in use */
-    int32_t view_groups;           /* views split into this many concurrently launched groups */
+    int32_t view_groups;           /* views split into this many groups, concurrent in the graph */
 } cr_batch_info;
 
 /* Copies the view list; validates each view as cr_set_surfaces /
@@ -372,8 +372,8 @@ cr_status cr_batch_draw(cr_batch* batch, void* stream);
  * stage's views longest-first by the measured entries per bin and per tile,
  * times every fine-stage workgroup shape with banded and round-robin tile
  * groups and both coarse workgroup sizes, then 1, 2 or 4 cost-balanced view
- * groups whose launch chains run concurrently (forked streams, parallel
- * graph branches), keeps the fastest, then captures the graph.  Bin size is chosen
+ * groups whose launch chains run concurrently (parallel graph branches; not
+ * with graphs off), keeps the fastest, then captures the graph.  Bin size is chosen
  * per view from its resolution (the smallest bins with at most 256 bins).
  * Surfaces of views without deferred clear are restored afterwards. */
 cr_status cr_batch_autotune(cr_batch* batch, void* stream);
@@ -388,7 +388,8 @@ cr_status cr_batch_reserve(cr_batch* batch, int32_t view, int64_t max_subtris, i
  * while those run. */
 cr_status cr_batch_set_buffers(cr_batch* batch, const void* const* vertices, const void* const* indices,
                                int32_t num_views);
-/* 0: launch the stages directly on each draw instead of replaying a graph. */
+/* 0: launch the stages directly on each draw, view groups one after the other,
+ * instead of replaying a graph. */
 cr_status cr_batch_use_graph(cr_batch* batch, int32_t enable);
 /* Sets the launch configuration the autotuner otherwise chooses (images do
  * not depend on it): fine tiles per workgroup (2, 4 or 8), fine tile groups
