@@ -736,12 +736,17 @@ void launchFinishBatch(const Params* views, int numViews, const Counters* devBas
 
 int coarseShapeFor(const Params& P) {
   if (P.coarseThreads == 256 || P.coarseThreads == 1024) return P.coarseThreads;
-  // A single draw leaves the GPU room for the large workgroups, which hide
-  // more of a long bin's latency (100k triangles at 1024^2 14.1 against 17.4
-  // us, 1M at 2048^2 37 against 72); with few entries per bin there is nothing
-  // to hide and the small ones' barriers are cheaper (12 triangles 12.0 against
-  // 10.9 us, 30k 13.1 against 12.2).  Batches tune it.
-  if (P.numTris < 32 * 1024) return 256;
+  // The stage's work is entries per bin, which only the draw itself counts: what
+  // is known before is that a bin has at most one per triangle (more only of
+  // clipped ones).  Where that is a single round, the small workgroups' barriers
+  // are cheaper by a microsecond (12 to 256 triangles at 256^2 to 1024x768, of 12
+  // pixels or of the whole view: 8.2 to 44 us against 9.5 to 44); in bins of 16x16
+  // tiles their four waves take longer over large boxes (2048^2, half the view's
+  // width: 12 triangles 12.7 us against 13.4, 64 24.0 against 19.3).  From the
+  // second round on the large ones hide more of each round's latency (2048^2,
+  // half the view's width: 512 triangles 91 us against 156, 20k 2.7 ms against
+  // 6.1; 1M small ones 37 against 72).  Batches tune it.
+  if (P.numTris <= (P.binLog2 < kBinLog2 ? 128 : 16)) return 256;
   return 1024;
 }
 
