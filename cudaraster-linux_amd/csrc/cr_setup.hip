@@ -540,15 +540,23 @@ __device__ __forceinline__ BinBox binBoxOf(const Params& P, uint4 h) {
   return b;
 }
 
-// Boxes of more bins than this are walked by their whole wave, 16 x 4 bins at
-// a time, instead of by their own lane bin by bin (a full-screen triangle's
-// 256 bins held its workgroup up for 150k cycles).
-constexpr int kCoopBins = 6;
-// A wave full of them is faster lane by lane, all boxes at once: 64 triangles
-// over the 230 bins of a 368x145 view, setup 36 against 78 us; the first 16 of
-// them the other way round, 44 against 30.  (Walking the bins of the boxes'
-// union took 59 for either and spilled registers.)
-constexpr int kCoopBoxes = 36;
+// A wave's wide boxes are walked by the whole wave, 16 x 4 bins at a time, one
+// box after another, instead of by their own lanes bin by bin, where the largest
+// has more than kCoopBins bins for each of them.  A box takes the wave as long as
+// three bins take the lanes if all waves of a workgroup have such boxes (their
+// additions to the masks collide), nine if one has.  Setup of 1024 triangles, k
+// of each 64 over 8 to 12 bins: lanes 2.6 us more than none for k = 4, 4 for 36,
+// wave 0.65 k; over 64 to 81 bins: lanes 19 and 27, wave 1.2 k; over 256: lanes 62
+// and 150, wave 2.7 k; 16 and 64 boxes of 230 bins in a single wave: lanes 34 and
+// 26, wave 20 and 68.
+constexpr int kCoopBins = 7;
+__device__ __forceinline__ bool coopBoxes(const BinBox& b) {
+  const int area = b.x0 <= b.x1 ? (b.x1 - b.x0 + 1) * (b.y1 - b.y0 + 1) : 0;
+  const uint64_t wide = __ballot(area > kCoopBins);
+  if (wide == 0) return false;
+  const int most = waveReduce(area, 0, [](int a, int c) { return max(a, c); });
+  return most > kCoopBins * (int)__popcll(wide) && area > kCoopBins;
+}
 
 // Calls f(bin, j) for every bin of lane j's box (j uniform).
 template <class F>
@@ -675,8 +683,7 @@ __device__ __forceinline__ void setupBinBody(Load&& load, const int chunk) {
       }
     }
     const uint64_t bit = 1ull << lane;
-    const bool wide = (bb.x1 - bb.x0 + 1) * (bb.y1 - bb.y0 + 1) > kCoopBins && bb.x0 <= bb.x1;
-    const bool big = wide && __popcll(__ballot(wide)) <= kCoopBoxes;
+    const bool big = coopBoxes(bb);
     if (!big) {
       for (int y = bb.y0; y <= bb.y1; y++)
         for (int x = bb.x0; x <= bb.x1; x++)
@@ -757,8 +764,7 @@ __device__ __forceinline__ void setupBinBody(Load&& load, const int chunk) {
       if (p < (uint32_t)P.maxBinEntries) P.binList[p] = e;
     };
     const uint4 e = make_uint4(slot, hv.x, hv.y, hv.z);
-    const bool wide = (bb.x1 - bb.x0 + 1) * (bb.y1 - bb.y0 + 1) > kCoopBins && bb.x0 <= bb.x1;
-    const bool big = wide && __popcll(__ballot(wide)) <= kCoopBoxes;
+    const bool big = coopBoxes(bb);
     if (!big) {
       const uint64_t lt = laneLt();
       for (int y = bb.y0; y <= bb.y1; y++)
