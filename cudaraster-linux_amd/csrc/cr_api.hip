@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -80,8 +81,13 @@ void clearValues(const float rgba[4], float depth, uint32_t* color, uint32_t* en
 }
 
 double clockTick(int device) {
-  int khz = 0;
-  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || khz <= 0) khz = 100000;
+  constexpr int kDevices = 64;
+  static std::atomic<int> rates[kDevices];     // kHz; 0: not asked for yet
+  int khz = device >= 0 && device < kDevices ? rates[device].load(std::memory_order_relaxed) : 0;
+  if (khz == 0) {
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || khz <= 0) khz = 100000;
+    if (device >= 0 && device < kDevices) rates[device].store(khz, std::memory_order_relaxed);
+  }
   return 1e-3 / khz;
 }
 
@@ -271,8 +277,10 @@ cr_status launchAll(cr_context* ctx, Params P, hipStream_t stream, bool own) {
   if (finish) launchFinish(P, ctx->hostCountersDev, stream);
   CR_HIP(ctx, hipGetLastError());
   if (own) ctx->countersClean = true;
-  if (!finish) ctx->counterBlock ^= 1;
-  ctx->lastEnd = finish ? nullptr : P.counters;
+  if (!finish) {
+    ctx->counterBlock ^= 1;
+    ctx->lastEnd = P.counters;
+  }
   if (P.prof)
     CR_HIP(ctx, hipMemcpyAsync(ctx->hostProf, P.prof, 2 * kProfCount * sizeof(unsigned long long),
                                hipMemcpyDeviceToHost, stream));
@@ -281,9 +289,9 @@ cr_status launchAll(cr_context* ctx, Params P, hipStream_t stream, bool own) {
   return CR_OK;
 }
 
-
 uint32_t recordCounters(cr_context* ctx) {
   const Counters& c = *ctx->hostCounters;
+  std::copy_n(c.stamp, (int)kStampCount, ctx->lastStamp);
   ctx->last.num_tris = ctx->numTris;
   ctx->last.num_subtris = c.numSubtris;
   ctx->last.bin_entries = c.binEntries;
@@ -378,7 +386,7 @@ cr_status cr_context_create(cr_context** out) {
   // a failed lookup is reported by that entry point, not here).
   if (e == hipSuccess) scratchInit(ctx->device);
   if (e == hipSuccess) e = ctx->counters.ensure(3 * sizeof(Counters));
-  if (e == hipSuccess) e = hipHostMalloc((void**)&ctx->hostCounters, sizeof(Counters), hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&ctx->hostCounters, 2 * sizeof(Counters), hipHostMallocDefault);
   if (e == hipSuccess)
     e = hipHostMalloc((void**)&ctx->hostProf, 2 * kProfCount * sizeof(unsigned long long), hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostGetDevicePointer((void**)&ctx->hostCountersDev, ctx->hostCounters, 0);
@@ -387,7 +395,7 @@ cr_status cr_context_create(cr_context** out) {
     cr_context_destroy(ctx);
     return fail(nullptr, CR_ERR_DEVICE, "cr_context_create: %s", hipGetErrorString(e));
   }
-  memset(ctx->hostCounters, 0, sizeof(Counters));
+  memset(ctx->hostCounters, 0, 2 * sizeof(Counters));
   memset(ctx->hostProf, 0, 2 * kProfCount * sizeof(unsigned long long));
   *out = ctx;
   return CR_OK;
@@ -404,6 +412,7 @@ cr_status cr_context_destroy(cr_context* ctx) {
   if (ctx->hostCounters) (void)hipHostFree(ctx->hostCounters);
   if (ctx->hostProf) (void)hipHostFree(ctx->hostProf);
   if (ctx->evPending) (void)hipEventDestroy(ctx->evPending);
+  if (ctx->statStream) (void)hipStreamDestroy(ctx->statStream);
   delete ctx;
   return CR_OK;
 }
@@ -615,6 +624,29 @@ cr_status cr_reserve(cr_context* ctx, int64_t maxSubtris, int64_t maxBin, int64_
   return CR_OK;
 }
 
+namespace {
+
+// The last of the fine waves' ends in the block ctx->lastEnd, of a draw that is
+// done: a copy per request, not per draw, on a stream of its own.  Nothing else is
+// waited for, and streams may be capturing (none of the draw's), which the
+// thread's relaxed mode is for.
+hipError_t readEnd(cr_context* ctx, uint64_t* end) {
+  hipError_t e = hipSetDevice(ctx->device);
+  if (e != hipSuccess) return e;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  e = hipThreadExchangeStreamCaptureMode(&mode);
+  if (e != hipSuccess) return e;
+  if (!ctx->statStream) e = hipStreamCreateWithFlags(&ctx->statStream, hipStreamNonBlocking);
+  Counters* c = ctx->hostCounters + 1;
+  if (e == hipSuccess) e = hipMemcpyAsync(c, ctx->lastEnd, sizeof(Counters), hipMemcpyDeviceToHost, ctx->statStream);
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->statStream);
+  if (e == hipSuccess) *end = *std::max_element(c->fineEnd, c->fineEnd + 8);
+  const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+  return e != hipSuccess ? e : back;
+}
+
+}  // namespace
+
 cr_status cr_get_stats(cr_context* ctx, cr_stats* out) {
   if (!ctx || !out) return fail(ctx, CR_ERR_INVALID, "cr_get_stats: NULL argument");
   memset(out, 0, sizeof(*out));
@@ -624,14 +656,11 @@ cr_status cr_get_stats(cr_context* ctx, cr_stats* out) {
   // setup kernel: its time is part of setup_time and bin_time is 0.  (A draw
   // without triangles has no setup stage and no setup stamp.)
   uint64_t s[kStampCount];
-  memcpy(s, ctx->hostCounters->stamp, sizeof(s));
-  if (ctx->lastEnd) {
-    // The fine stage's workgroups left their ends in the device's block, which
-    // the next draw clears (a copy per request, not per draw).
-    Counters c;
-    CR_HIP(ctx, hipSetDevice(ctx->device));
-    CR_HIP(ctx, hipMemcpy(&c, ctx->lastEnd, sizeof(c), hipMemcpyDeviceToHost));
-    s[kStampEnd] = *std::max_element(c.fineEnd, c.fineEnd + 8);
+  std::copy_n(ctx->pending ? ctx->hostCounters->stamp : ctx->lastStamp, (int)kStampCount, s);
+  if (s[kStampEnd] == 0 && ctx->lastEnd) {
+    // The draw had no finish kernel: the fine stage's waves left their ends in
+    // the device's block, which the next draw clears.
+    CR_HIP(ctx, readEnd(ctx, &s[kStampEnd]));
   }
   const double tick = clockTick(ctx->device);
   auto seconds = [&](uint64_t from, uint64_t to) {

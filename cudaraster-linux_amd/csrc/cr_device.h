@@ -91,7 +91,7 @@ struct Counters {
   uint64_t fragments;      // (subtriangle, pixel) pairs with >= 1 covered sample
   uint64_t visibleSubtris; // subtriangles that survive setup (counting draws only)
   uint64_t stamp[kStampCount];   // wall clock at the stages' starts and the draw's end (0: stage not run)
-  uint64_t fineEnd[8];           // per XCD: wall clock at a last fine workgroup's end (draws without a finish kernel)
+  uint64_t fineEnd[8];           // per XCD: wall clock at a last fine wave's end (draws without a finish kernel)
   uint64_t pad[26 - kStampCount - 8];
 };
 static_assert(sizeof(Counters) == 256, "counter block");

@@ -261,7 +261,7 @@ __device__ __forceinline__ int xcdGroup(int groups) {
 
 // A plain draw's end, by workgroups of the fine stage themselves: the first
 // one hands the counters to the host (pinned memory, visible when the kernel
-// has ended) and clears the next draw's; each notes its end.
+// has ended) and clears the next draw's; every wave notes its end.
 __device__ __forceinline__ void handOver(const Params& P, int group) {
   static_assert(sizeof(Counters) == 64 * 4, "one word per lane");
   if (group != 0 || P.hostCounters == nullptr || threadIdx.x >= 64) return;
@@ -276,13 +276,15 @@ __device__ __forceinline__ void handOver(const Params& P, int group) {
   if (P.nextCounters != nullptr) reinterpret_cast<uint32_t*>(P.nextCounters)[i] = 0;
 }
 // (Called by kernels whose first argument is the draw's Params; it reads the
-// two pointers there again, so that nothing is kept in registers for it.)
+// two pointers there again, so that nothing is kept in registers for it.  Waves
+// of an XCD share a word: the last store to land stays, a store's latency at
+// most before the last end.)
 __device__ __forceinline__ void noteEnd() {
   using Arg = const __attribute__((address_space(4))) uint8_t;
   Arg* args = (Arg*)__builtin_amdgcn_kernarg_segment_ptr();
   __asm__ volatile("" : "+s"(args));
   using Word = const __attribute__((address_space(4))) uint64_t;
-  if (*(Word*)(args + offsetof(Params, hostCounters)) == 0 || threadIdx.x != 0) return;
+  if (*(Word*)(args + offsetof(Params, hostCounters)) == 0 || (threadIdx.x & 63) != 0) return;
   Counters* c = (Counters*)(uintptr_t)*(Word*)(args + offsetof(Params, counters));
   makeGlobal(c);
   c->fineEnd[blockIdx.x & 7] = wall_clock64();

@@ -99,8 +99,8 @@ cr_status fail(cr_context* ctx, cr_status st, const char* fmt, ...);
 // (CudaRaster.cpp:174-179, base/Math.cpp:41-48, cuda/Util.hpp:290-298).
 void clearValues(const float rgba[4], float depth, uint32_t* color, uint32_t* encodedDepth);
 
-// Seconds per tick of the device's wall clock (asked for when times are: the
-// query takes tens of microseconds).
+// Seconds per tick of the device's wall clock (asked for once per device, when
+// times are: the query takes tens of microseconds).
 double clockTick(int device);
 
 // setPixelPipe's checks of a pipe descriptor (CudaRaster.cpp:183-216).
@@ -141,7 +141,8 @@ crhip::Params makeParams(cr_context* ctx, const Geometry& g, int32_t numChunks, 
 // ctx->hostCounters.  own: P.counters is the context's block of its next draw;
 // else a block that other draws may have left in use, cleared first.
 cr_status launchAll(cr_context* ctx, crhip::Params P, hipStream_t stream, bool own);
-// Copies the read-back counters into ctx->last; returns their overflow bits.
+// Copies the read-back counters and stage stamps into ctx->last and
+// ctx->lastStamp; returns the overflow bits.
 uint32_t recordCounters(cr_context* ctx);
 // Looks up this device's copy of the no-allocation draw's fixed scratch
 // array (once per device; the device must be current).
@@ -181,11 +182,15 @@ struct cr_context {
   crhost::DevBuf tileStart, tileCount, tileList, tileSegNext, tileFrags, chunkSubtris;
   crhost::DevBuf counters, profBuf;          // counters: two blocks for draws in turn, one for captured draws
   crhost::DevBuf interpAcc;                  // fixed-point gradient accumulators (deterministic backward)
-  crhip::Counters* hostCounters = nullptr;   // pinned, written by the draw's finish kernel
+  // Pinned: the last draw's counters, written by its fine stage or its finish
+  // kernel, then a block that cr_get_stats reads into.
+  crhip::Counters* hostCounters = nullptr;
   crhip::Counters* hostCountersDev = nullptr;   // its device address
   bool countersClean = false;                // the last draw was queued whole: it leaves the next block cleared
   int counterBlock = 0;                      // which of the two blocks in `counters` the next draw uses
-  const crhip::Counters* lastEnd = nullptr;  // the last draw's device block when it holds the end stamps
+  const crhip::Counters* lastEnd = nullptr;  // device block with the fine waves' ends, of the last draw that left them there
+  uint64_t lastStamp[crhip::kStampCount] = {};  // the last completed draw's stage stamps (no end: see lastEnd)
+  hipStream_t statStream = nullptr;   // cr_get_stats' copies
   unsigned long long* hostProf = nullptr;    // pinned, 2 * kProfCount
   cr_profile_counters lastProf{};
   bool lastProfiled = false;                 // the last launch recorded profile counters

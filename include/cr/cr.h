@@ -137,7 +137,8 @@ typedef struct cr_pipe_desc {
 
 /* CudaRaster::Stats (CudaRaster.hpp:45-51): seconds per stage of the last
  * draw, from device clock stamps.  Triangle setup and binning run as one kernel:
- * setup_time covers both and bin_time is 0. */
+ * setup_time covers both and bin_time is 0.  fine_time lasts to the end of the
+ * last wave, within about a microsecond. */
 typedef struct cr_stats {
     float setup_time;
     float bin_time;
