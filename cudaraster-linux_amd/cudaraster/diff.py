@@ -92,10 +92,11 @@ class InterpolateViews:
             @staticmethod
             def backward(ctx, grad_out, _grad_ids):
                 n = ctx.n
-                if grad_out is None:
-                    return (None,) * (2 + 3 * n)
                 ids, *tensors = ctx.saved_tensors
                 pos, attr, tris = tensors[:n], tensors[n:2 * n], tensors[2 * n:3 * n]
+                if grad_out is None:         # an undefined gradient of the images: zeros
+                    zeros = [torch.zeros_like(x) for x in (*pos, *attr)]
+                    return (None, None, *zeros, *([None] * n))
                 gp, ga = ctx.raster._interpolate_views_backward(pos, attr, tris, ids, grad_out.contiguous())
                 return (None, None, *gp, *ga, *([None] * n))
 
