@@ -79,20 +79,22 @@ __device__ __forceinline__ bool pixelTriangle(const InterpGeom& G, const InterpV
   return true;
 }
 
-constexpr int kFwdTile = 16;
+constexpr int kFwdThreads = 256;
 
-// One lane per pixel, one 16x16-pixel tile per workgroup, one grid layer per
-// view.  Bound by the gathers of vertices: a tile's pixels share them in the
-// CU's cache, a row's hardly do.  16 views of 200k triangles, 512x512, 8
-// channels: 107 us in rows of 256 pixels, 82 in tiles (86 with every lane's
-// channels fetched ahead of its barycentrics).
+// One lane per pixel, one W x (256 / W) pixel tile per workgroup, one grid layer
+// per view.  Bound by the gathers of vertices where triangles are small: a
+// tile's pixels share them in the CU's cache, a row's hardly do.  16 views of
+// 200k triangles, 512x512, 8 channels: 97 us in rows of 256 pixels, 90 in 64 x 4,
+// 83 in 32 x 8, 82 in 16 x 16.  Bound by the stores where they are large: a
+// row's are longer runs.  1024x1024, 8k triangles, 24 channels: 46 us in rows, 56 in
+// 64 x 4, 55 in 32 x 8, 62 in 16 x 16.
 // vec4: C % 4 == 0 and attr / out 16-byte aligned, so channels move as
 // float4.
-template <int N>
-__global__ void __launch_bounds__(kFwdTile * kFwdTile) interpForwardKernel(const InterpGeom G, const InterpTable<N> T) {
+template <int N, int W>
+__global__ void __launch_bounds__(kFwdThreads) interpForwardKernel(const InterpGeom G, const InterpTable<N> T) {
   const InterpView& V = T.v[N == 1 ? 0 : blockIdx.z];
-  const int x = (int)(blockIdx.x * kFwdTile + threadIdx.x % kFwdTile);
-  const int y = (int)(blockIdx.y * kFwdTile + threadIdx.x / kFwdTile);
+  const int x = (int)(blockIdx.x * W + threadIdx.x % W);
+  const int y = (int)(blockIdx.y * (kFwdThreads / W) + threadIdx.x / W);
   if (x >= G.width || y >= G.height) return;
   const int64_t p = (int64_t)y * G.width + x;
   const int C = G.numChannels;
@@ -591,11 +593,23 @@ __global__ void __launch_bounds__(256) fixedToFloatKernel(const InterpTable<N> T
   }
 }
 
+template <int W, int N>
+static void forwardTiles(const InterpGeom& G, const InterpTable<N>& T, int n, hipStream_t stream) {
+  constexpr int H = kFwdThreads / W;
+  hipLaunchKernelGGL((interpForwardKernel<N, W>), dim3((unsigned)((G.width + W - 1) / W),
+                     (unsigned)((G.height + H - 1) / H), (unsigned)n), dim3(kFwdThreads), 0, stream, G, T);
+}
+
 template <int N>
 static void forwardViews(const InterpGeom& G, const InterpTable<N>& T, int n, hipStream_t stream) {
-  hipLaunchKernelGGL((interpForwardKernel<N>), dim3((unsigned)((G.width + kFwdTile - 1) / kFwdTile),
-                     (unsigned)((G.height + kFwdTile - 1) / kFwdTile), (unsigned)n), dim3(kFwdTile * kFwdTile), 0,
-                     stream, G, T);
+  // Tiles from one triangle in four pixels on.  1024x1024, rows against 32 x 8: a
+  // mesh of 512x512 vertices (a triangle in two pixels), 1 channel 10.1 and 10.0
+  // us, 16 34.8 and 29.9, 20 54.9 and 48.7; 300x300 (one in six), 24 channels 53.7 and
+  // 59.3; 65x65, 1 channel 10.3 and 10.4, 16 25.3 and 26.2, 20 33.3 and 38.9.
+  int64_t tris = 0;
+  for (int v = 0; v < n; v++) tris += T.v[v].numTris;
+  if (tris * 4 >= (int64_t)G.width * G.height * n) forwardTiles<32>(G, T, n, stream);
+  else forwardTiles<256>(G, T, n, stream);
 }
 
 template <int N>
