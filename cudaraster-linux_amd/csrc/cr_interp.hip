@@ -218,19 +218,21 @@ __device__ __forceinline__ void loadChannels(const float* __restrict__ p, int n,
 // two) that starts out all kNoKey.  Consecutive keys start at consecutive
 // slots; the multiple of the key's high part keeps keys that are a power of
 // two apart (the rows of a grid) from starting at the same one.  Rows that do
-// fall on one another are taken apart by steps that 32 consecutive keys share, so
-// that they stay together (odd: they reach every slot; the high bits of a product
-// with 2^32 over the golden ratio).  In steps of one they queued up behind each
-// other: 512x512, meshes of 988x988, 1000x1000 and 717x717 vertices, 3 channels
-// 169, 145 and 55 us, now 60, 63 and 35.
+// fall on one another are taken apart by jumps of 1, 3, 6, ... steps (which reach
+// every slot when the step is odd), the step shared by 32 consecutive keys, so
+// that they stay together (the high bits of a product with 2^32 over the golden
+// ratio).  In steps of one the rows queued up behind each other, and with jumps of
+// one step some pairs of rows still did: 512x512, meshes of 988x988, 1000x1000
+// and 717x717 vertices, 3 channels 169, 145 and 55 us, 60, 63 and 35, now 59, 61 and
+// 34; 256x256, 257x257 17, 26 and 18.
 template <int SLOTS>
 __device__ __forceinline__ uint32_t hashSlot(uint32_t* table, uint32_t key) {
   uint32_t h = (key + (key / SLOTS) * 37u) & (SLOTS - 1);
   const uint32_t step = ((key >> 5) * 0x9E3779B1u >> 20) | 1u;
-  for (;;) {
+  for (uint32_t jump = step;; jump += step) {
     const uint32_t old = atomicCAS(&table[h], kNoKey, key);
     if (old == kNoKey || old == key) return h;
-    h = (h + step) & (SLOTS - 1);
+    h = (h + jump) & (SLOTS - 1);
   }
 }
 
