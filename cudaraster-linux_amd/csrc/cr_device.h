@@ -486,7 +486,7 @@ void launchVertexPassthrough(const float* modelPos, int64_t numVertices, const f
                              int64_t outStride, hipStream_t stream);
 void launchInterpForward(const InterpGeom& G, const InterpView* views, int numViews, hipStream_t stream);
 // gradPos (4 per vertex) and gradAttr (C per vertex) are overwritten.  The
-// per-(tile, triangle) FP64 sums are added with FP32 atomics (acc null in
+// per-(tile, vertex) FP64 sums are added with FP32 atomics (acc null in
 // every view), or, bit-reproducibly, as 128-bit fixed-point integers in each
 // view's acc (2 * (4 + C) * V 64-bit words) rounded to FP32 at the end.
 void launchInterpBackward(const InterpGeom& G, const InterpView* views, int numViews, hipStream_t stream);
