@@ -469,7 +469,9 @@ cr_status settleOverflow(cr_batch* b, hipStream_t stream) {
 // run, the counters neither cleared nor the moved buffers written).
 cr_status refuseCapture(cr_batch* b, hipStream_t stream) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  CR_HIP(b->ctx, hipStreamIsCapturing(stream, &cap));
+  const hipError_t e = hipStreamIsCapturing(stream, &cap);
+  if (e != hipSuccess) (void)hipGetLastError();    // (the null stream beside a capturing one; not for the next draw to find)
+  CR_HIP(b->ctx, e);
   if (cap != hipStreamCaptureStatusNone)
     return fail(b->ctx, CR_ERR_DEVICE, "batch: the draw waits for its counters, which a capturing stream cannot");
   return CR_OK;
